@@ -307,3 +307,21 @@ def test_sht_round_trip_config2_full_batch():
     S3, T3 = mix.spat_to_sphertor(vtm, vpm)
     assert float((S3 - S2).abs().max() / ss) < 1e-5
     assert float((T3 - T2).abs().max() / T.abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed", "mixed_bf16x3"])
+def test_sht_batch_wider_than_the_radial_grid(precision):
+    """A transform of more columns than the resolution has radial levels reads no
+    radial profile: each column equals its transform alone."""
+    torch = _torch()
+    from magic_amd.params import Params
+    from magic_amd.device import Resolution
+    from magic_amd.sht import SHT
+    res = Resolution(Params({"l_max": 16, "n_r_max": 9}))
+    sht = SHT(res, precision)
+    rng = np.random.default_rng(4)
+    x = [torch.from_numpy(rng.standard_normal((res.L, 40)) + 0j).cuda() for _ in range(3)]
+    wide = sht.torpol_to_spat(*x)
+    for c in (0, 9, 39):
+        one = sht.torpol_to_spat(*[v[:, c].contiguous() for v in x])
+        assert all(torch.equal(a[c], b) for a, b in zip(wide, one))

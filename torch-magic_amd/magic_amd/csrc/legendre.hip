@@ -159,7 +159,6 @@ __global__ __launch_bounds__(64 * WAVES, 3) void k_syn(SynArgs a, int n_m) {
   const int sg = scol ? sbc / a.B : 0;
   const int sb = scol ? sbc - sg * a.B : 0;
   const long soff = 2L * sb + (cw & 1);
-  const double sor2 = scol ? a.or2[sb] : 0.0;
   // this thread's input pointers (column offset folded in) and modes, resolved
   // once: per-lane selection inside the chunk loop would re-read the argument
   // block through memory on every chunk
@@ -173,6 +172,9 @@ __global__ __launch_bounds__(64 * WAVES, 3) void k_syn(SynArgs a, int n_m) {
     if (f == 2) sx2 = in.x2 + soff;
     smodes |= in.mode << (2 * f);
   }
+  // or2 (a.B entries) is read for the fields that use it only: other inputs may have
+  // more columns than the radial grid has levels
+  const double sor2 = (scol && ((smodes >> 4) & 3) == 2) ? a.or2[sb] : 0.0;
   acc_t acc[NA];  // acc[(5p + q) * NCT + ct] (vector), acc[p * NCT + ct] (scalar)
 #pragma unroll
   for (int q = 0; q < NA; ++q) acc[q] = (acc_t){0, 0, 0, 0};

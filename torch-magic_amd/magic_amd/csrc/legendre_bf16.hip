@@ -101,7 +101,6 @@ __global__ __launch_bounds__(256, 2) void k_syn_bf(SynArgs a, int n_m) {
   const int sg = scol ? sbc / a.B : 0;
   const int sb = scol ? sbc - sg * a.B : 0;
   const long soff = 2L * sb + (cw & 1);
-  const double sor2 = scol ? a.or2[sb] : 0.0;
   const double* sx1[NF];
   const double* sx2 = nullptr;
   int smodes = 0;
@@ -112,6 +111,9 @@ __global__ __launch_bounds__(256, 2) void k_syn_bf(SynArgs a, int n_m) {
     if (f == 2) sx2 = in.x2 + soff;
     smodes |= in.mode << (2 * f);
   }
+  // or2 (a.B entries) is read for the fields that use it only: other inputs may have
+  // more columns than the radial grid has levels
+  const double sor2 = (scol && ((smodes >> 4) & 3) == 2) ? a.or2[sb] : 0.0;
   float4_t acc[NA];
 #pragma unroll
   for (int q = 0; q < NA; ++q) acc[q] = (float4_t){0, 0, 0, 0};
