@@ -34,7 +34,9 @@ extern "C" {
  * northern nodes, written into the synthesis / analysis table layouts.
  * Replaces plms.build_plm_matrices (plms.py:158-186) and the padded/bucketed
  * SHT matrices of sht.py:84-289.  mp_info[(m*2+p)*4 + {0..3}] =
- * {K, syn_off, ana_off, K16} for parity p = (l-m)%2. */
+ * {K, syn_off, ana_off, K16} for parity p = (l-m)%2, K degrees up to l_max; the P_lm
+ * tables hold the degree l_max + 1 too (one row more where its parity is p).
+ * synP ends with 48 Hp finite values past the last row that are read and unused. */
 int mh_plm_tables(int l_max, int n_m, int minc, int H, int Hp, const double* cos_t, const double* sin_t,
                   const double* wgt, const int* mp_info, double* synP, double* synD,
                   double* anaW, double* anaWd, void* stream);
@@ -62,11 +64,17 @@ typedef struct {
                 mh_tables_to_bf16), BF16 MFMA on the products of planes i, j with
                 i + j < prec (3 or 6 products), FP32 accumulation */
   int fprec; /* 0: F holds doubles; 1: F holds floats (FP32 Fourier buffers, needs prec >= 1) */
-  int waves; /* waves per workgroup (16 theta pairs each): 0 = default (4), 4 or 6 (prec <= 1) */
+  int waves; /* waves per workgroup (16 theta pairs each): 0 = default (4), 4 or 6 (prec 1;
+                prec 0 chooses by itself) */
   int nct;   /* column tiles of 8 complex columns per workgroup: 0/1, or 2 (prec >= 1, vector) */
   int minc;  /* azimuthal symmetry: mode index m holds the order m * minc (0 reads as 1) */
   const int* mp16; /* prec >= 2: per (m, parity) {K32, synthesis offset, analysis offset, 0}
                       of the bf16 tables (elements) */
+  const double* lcf; /* prec 0: per degree l = m .. l_max + 1 of each order the four values
+                        (l - 1) c_l, (l + 2) c_{l+1}, (l + 1) c_l, l c_{l+1} with c_l = sqrt((l^2 -
+                        m^2) / (4 l^2 - 1)), row lm_start[m] + m + (l - m) (m: mode index in the
+                        first two) */
+  int l_max, pad1;   /* prec 0 (the x1, x2 and F rows must lie on 16 bytes) */
 } MhSynArgs;
 
 /* Legendre synthesis on FP64 MFMA: scalar (vector=0) replaces the bmm part of
@@ -87,7 +95,9 @@ typedef struct {
   const int* lm_start;
   const double* anaW;
   const double* anaWd;
-  const int* tiles; /* (m, p, k0) triples, k0 in steps of 96 degrees (one workgroup each) */
+  const int* tiles; /* (m, p, k0) triples, one workgroup each, k0 in steps of 16 * waves degrees
+                       (prec 0: (m, count << 16 | number, k0), the windows of 60 indices k = (l - m
+                       - p) / 2 of one order together, each for both parities p) */
   int ntiles;
   int prec;  /* as MhSynArgs.prec (anaW/anaWd hold floats for 1, the bf16 tables for 2, 3) */
   int fprec; /* as MhSynArgs.fprec: F holds floats for 1 (needs prec >= 1) */
@@ -95,6 +105,9 @@ typedef struct {
                 must hold 16 * waves degrees */
   int minc;  /* as MhSynArgs.minc */
   const int* mp16; /* prec >= 2: as MhSynArgs.mp16 */
+  const double* lcf; /* prec 0: as MhSynArgs.lcf */
+  int l_max;
+  int pad1;
 } MhAnaArgs;
 
 /* Legendre analysis on FP64 MFMA: scalar replaces the bmm part of scal_to_SH

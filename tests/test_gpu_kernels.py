@@ -325,3 +325,30 @@ def test_sht_batch_wider_than_the_radial_grid(precision):
     for c in (0, 9, 39):
         one = sht.torpol_to_spat(*[v[:, c].contiguous() for v in x])
         assert all(torch.equal(a[c], b) for a, b in zip(wide, one))
+
+
+@pytest.mark.parametrize("l_max,B,minc", [(126, 25, 1), (20, 8, 1), (48, 9, 2)])
+def test_fp64_transforms_at_tile_edges(l_max, B, minc):
+    """FP64 vector and scalar transforms where the work split has edges: orders
+    with one and with two analysis windows (l_max = 126: 121 or 122 degrees at m =
+    6 and 5), an odd number of theta tiles, column counts at and past a tile of 8
+    and 24; against the oracle to rounding (sums of up to l_max terms)."""
+    torch = _torch()
+    from magic_amd.params import Params
+    from magic_amd.device import Resolution
+    from magic_amd.sht import SHT
+    res = Resolution(Params({"l_max": l_max, "n_r_max": 9, "minc": minc}))
+    sht, osht = SHT(res), _oracle_sht(l_max, minc)
+    Q, S, T = (_rand_spec(res.L, B, res.maps, k) for k in (1, 2, 3))
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    tol = 4 * l_max * np.finfo(float).eps
+    grids = osht.torpol_to_spat(Q, S, T)
+    for a, b in zip(sht.torpol_to_spat(dev(Q), dev(S), dev(T)), grids):
+        assert np.abs(a.cpu().numpy() - b).max() < tol * np.abs(b).max()
+    sc = osht.scal_to_spat(Q)
+    assert np.abs(sht.scal_to_spat(dev(Q)).cpu().numpy() - sc).max() < tol * np.abs(sc).max()
+    back = osht.scal_to_SH(sc)
+    assert np.abs(sht.scal_to_SH(dev(sc)).cpu().numpy() - back).max() < tol * np.abs(back).max()
+    for a, b in zip(sht.spat_to_sphertor(dev(grids[1]), dev(grids[2])),
+                    osht.spat_to_sphertor(grids[1], grids[2])):
+        assert np.abs(a.cpu().numpy() - b).max() < tol * np.abs(b).max()

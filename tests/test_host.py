@@ -456,3 +456,27 @@ def test_finite_difference_host_operators_match_oracle(cfg):
     s0, p0 = fdstep.conduction_state(p, rad, prof)
     os0, op0 = ofd.ps_cond(op, orr, fm, oprof)
     assert np.abs(s0 - os0).max() < 1e-12 and np.abs(p0 - op0).max() < 1e-12 * np.abs(op0).max()
+
+
+@pytest.mark.parametrize("l_max,minc", [(16, 1), (126, 1), (383, 1), (240, 4)])
+def test_fp64_analysis_windows_write_every_degree_once(l_max, minc):
+    """Windows of 60 degree indices k, four waves of 16 with 15 between their
+    starts: parity 0 takes k after its first one (all at the start of an order),
+    parity 1 all but its last; each degree l - m = 2 k + p <= l_max is written by
+    one wave, and a wave that starts past the last degree writes none."""
+    p = Params({"l_max": l_max, "minc": minc})
+    lay = grid.sht_layout(p, grid.lm_maps(p))
+    tiles = lay["ana_tiles_f64"].reshape(-1, 3)
+    for mi in range(p.n_m):
+        n = l_max + 1 - mi * minc
+        mine = tiles[tiles[:, 0] == mi]
+        assert [t[1] & 0xffff for t in mine] == list(range(len(mine)))
+        assert np.all(mine[:, 1] >> 16 == len(mine)) and np.all(mine[:, 2] == 60 * np.arange(len(mine)))
+        rows = []
+        for k0 in mine[:, 2]:
+            for kb in k0 + 15 * np.arange(4):
+                got = [2 * (kb + i) + q for q in (0, 1) for i in range(16)
+                       if 2 * (kb + i) + q < n and (i < 15 if q else (i > 0 or kb == 0))]
+                assert not got or kb == 0 or 2 * kb + 1 < n
+                rows += got
+        assert sorted(rows) == list(range(n))

@@ -33,7 +33,7 @@ class SynArgs(C.Structure):
     _fields_ = [("in_", (SynIn * 3) * 4), ("ngroups", I), ("B", I), ("ldx", I), ("H", I),
                 ("Hp", I), ("mp_info", P), ("lm_start", P), ("synP", P), ("synD", P),
                 ("or2", P), ("F", P), ("c_stride", L), ("m_stride", L), ("Bout", I), ("prec", I), ("fprec", I), ("waves", I), ("nct", I), ("minc", I),
-                ("mp16", P)]
+                ("mp16", P), ("lcf", P), ("l_max", I), ("pad1", I)]
 
 
 class AnaArgs(C.Structure):
@@ -41,7 +41,7 @@ class AnaArgs(C.Structure):
                 ("cf1", I * 3), ("cf2", I * 3), ("pad0", I), ("outS", P * 3), ("outT", P * 3),
                 ("ldo", I), ("H", I), ("Hp", I), ("n_m", I), ("mp_info", P), ("lm_start", P),
                 ("anaW", P), ("anaWd", P), ("tiles", P), ("ntiles", I), ("prec", I), ("fprec", I), ("waves", I),
-                ("minc", I), ("mp16", P)]
+                ("minc", I), ("mp16", P), ("lcf", P), ("l_max", I), ("pad1", I)]
 
 
 class FftArgs(C.Structure):

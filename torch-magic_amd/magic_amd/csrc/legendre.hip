@@ -1,9 +1,12 @@
-// Legendre tables and MFMA Legendre synthesis / analysis (FP64, or FP32 with
-// FP32 accumulation) for gfx950.
+// Legendre tables and the FP32 MFMA Legendre synthesis / analysis (FP32 tables
+// and accumulation, inputs rounded to FP32 as they are loaded) for gfx950.  FP64:
+// legendre_f64.hip; BF16 split: legendre_bf16.hip.
 //
 // Table layouts (per azimuthal order m and parity p = (l-m)%2, l = m+p+2k):
-//   synthesis  syn[m][p][k][j]  (k < K4 = roundup(K,4), j < Hp)  j fastest
-//   analysis   ana[m][p][j][k]  (j < Hp, k < K16 = roundup(K,16)) k fastest
+//   synthesis  syn[m][p][k][j]  (k < roundup(K+,4), j < Hp)  j fastest
+//   analysis   ana[m][p][j][k]  (j < Hp, k < K16 = roundup(K+,16)) k fastest
+// K is the number of degrees <= l_max of that parity and K+ that of degrees <=
+// l_max + 1 (the P_lm tables hold the extra degree, see legendre_f64.hip).
 // j indexes the northern Gauss nodes (theta pairs), Hp = roundup(H,32).
 // mp_info[(m*2+p)*4 + {0,1,2,3}] = {K, syn_off, ana_off, K16}.
 //
@@ -37,7 +40,7 @@ __global__ void k_plm_tables(int l_max, int minc, int H, int Hp, const double* _
     pmm = 0.0;
   }
   double pm1 = 0.0, p0 = pmm;  // P_{l-1}, P_l (unnormalised)
-  for (int l = m; l <= l_max; ++l) {
+  for (int l = m; l <= l_max + 1; ++l) {  // P up to l_max + 1, sin(theta) dP up to l_max
     const int L1 = l + 1;  // P_{l+1}
     double p1;
     if ((L1 - m) * (L1 + m) > 0) {
@@ -57,11 +60,13 @@ __global__ void k_plm_tables(int l_max, int minc, int H, int Hp, const double* _
     const int p = (l - m) & 1, k = (l - m) >> 1;
     const int* info = mp_info + (mi * 2 + p) * 4;
     const long so = (long)info[1] + (long)k * Hp + j;
-    synP[so] = P;
-    synD[so] = dP;
     const long ao = (long)info[2] + (long)j * info[3] + k;
+    synP[so] = P;
     anaW[ao] = w2pi * P;
-    anaWd[ao] = w2pi * dP;
+    if (l <= l_max) {
+      synD[so] = dP;
+      anaWd[ao] = w2pi * dP;
+    }
     pm1 = p0;
     p0 = p1;
   }
@@ -80,31 +85,6 @@ extern "C" int mh_plm_tables(int l_max, int n_m, int minc, int H, int Hp, const 
 
 // ---------------------------------------------------------------- synthesis
 
-__device__ __forceinline__ double syn_load(const SynIn& in, long lm, int l, int b, int reim,
-                                           int ldx, const double* or2) {
-  const long off = lm * 2 * (long)ldx + 2 * b + reim;
-  const double dl = (double)l * (double)(l + 1);
-  if (in.mode == 0) return in.x1[off];
-  if (in.mode == 1) return dl * in.x1[off];
-  return -in.x1[off] + or2[b] * dl * in.x2[off];
-}
-
-// Element type of the Legendre contraction: FP64 (16x16x4 f64 MFMA) or FP32
-// (16x16x4 f32 MFMA, FP32 accumulation; tables stored in FP32, inputs rounded
-// to FP32 as they are loaded).
-template <typename T> struct Mfma;
-template <> struct Mfma<double> {
-  typedef double4_t acc_t;
-  static __device__ __forceinline__ acc_t run(double a, double b, acc_t c) { return mfma_f64(a, b, c); }
-  // row of the 16x16 accumulator held in element v of a lane
-  static __device__ __forceinline__ int row(int lane, int v) { return mfma_row(lane, v); }
-};
-template <> struct Mfma<float> {
-  typedef float4_t acc_t;
-  static __device__ __forceinline__ acc_t run(float a, float b, acc_t c) { return mfma_f32(a, b, c); }
-  static __device__ __forceinline__ int row(int lane, int v) { return mfma_row_f32(lane, v); }
-};
-
 // Synthesis, one workgroup per (order m, 96 theta pairs, 8 complex columns).
 // Columns of the groups are laid side by side (column bc is batch column
 // bc % B of group bc / B, which is also its column in F).  The input tile of
@@ -118,13 +98,13 @@ template <> struct Mfma<float> {
 constexpr int kSynWavesDefault = 4, kSynDepth = 4;
 
 // NCT column tiles of 8 complex columns per workgroup: every table operand
-// feeds NCT MFMAs.  Two are instantiated for the FP32 vector synthesis (its
-// 20 accumulators fit; FP64 would not), chosen by the tuner.
-template <bool VEC, typename T, int NCT, typename FT, int WAVES>
+// feeds NCT MFMAs.  Two are instantiated for the vector synthesis (its 20
+// accumulators fit), chosen by the tuner.
+template <bool VEC, int NCT, typename FT, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, 3) void k_syn(SynArgs a, int n_m) {
   FT* const Fo = reinterpret_cast<FT*>(a.F);  // Fourier buffer elements (double or float)
-  typedef Mfma<T> MF;
-  typedef typename MF::acc_t acc_t;
+  typedef float T;
+  typedef float4_t acc_t;
   constexpr int NF = VEC ? 3 : 1;           // fields per group (Q, S, T)
   constexpr int NT = 64 * WAVES;            // threads
   constexpr int kSynJ = 16 * WAVES;         // theta pairs per workgroup
@@ -255,15 +235,15 @@ __global__ __launch_bounds__(64 * WAVES, 3) void k_syn(SynArgs a, int n_m) {
           const int cc = 16 * ct + col;
           const T xq = xs[buf][0][kr][cc];
           if (!VEC) {
-            acc[p * NCT + ct] = MF::run(aP, xq, acc[p * NCT + ct]);
+            acc[p * NCT + ct] = mfma_f32(aP, xq, acc[p * NCT + ct]);
           } else {
             const T xsv = xs[buf][1][kr][cc];
             const T xt = xs[buf][2][kr][cc];
-            acc[(5 * p + 0) * NCT + ct] = MF::run(aP, xq, acc[(5 * p + 0) * NCT + ct]);   // P Q
-            acc[(5 * p + 1) * NCT + ct] = MF::run(aP, xt, acc[(5 * p + 1) * NCT + ct]);   // P T
-            acc[(5 * p + 2) * NCT + ct] = MF::run(aP, xsv, acc[(5 * p + 2) * NCT + ct]);  // P S
-            acc[(5 * p + 3) * NCT + ct] = MF::run(aD, xsv, acc[(5 * p + 3) * NCT + ct]);  // dP S
-            acc[(5 * p + 4) * NCT + ct] = MF::run(aD, xt, acc[(5 * p + 4) * NCT + ct]);   // dP T
+            acc[(5 * p + 0) * NCT + ct] = mfma_f32(aP, xq, acc[(5 * p + 0) * NCT + ct]);   // P Q
+            acc[(5 * p + 1) * NCT + ct] = mfma_f32(aP, xt, acc[(5 * p + 1) * NCT + ct]);   // P T
+            acc[(5 * p + 2) * NCT + ct] = mfma_f32(aP, xsv, acc[(5 * p + 2) * NCT + ct]);  // P S
+            acc[(5 * p + 3) * NCT + ct] = mfma_f32(aD, xsv, acc[(5 * p + 3) * NCT + ct]);  // dP S
+            acc[(5 * p + 4) * NCT + ct] = mfma_f32(aD, xt, acc[(5 * p + 4) * NCT + ct]);   // dP T
           }
         }
         const long tn = (long)min(t + D, nsteps - 1) * tstep;
@@ -300,7 +280,7 @@ __global__ __launch_bounds__(64 * WAVES, 3) void k_syn(SynArgs a, int n_m) {
   auto A = [&](int q, int i) { return (double)acc[q * NCT + ct][i]; };
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int j = j0 + MF::row(lane, i);
+    const int j = j0 + mfma_row_f32(lane, i);
     const bool st = bval && (j < a.H);
     const long oN = fidx(a.c_stride, a.m_stride, a.Bout, 0, m, 2 * j, bo) + reim;
     const long oS = fidx(a.c_stride, a.m_stride, a.Bout, 0, m, 2 * j + 1, bo) + reim;
@@ -349,25 +329,23 @@ extern "C" int mh_leg_synth(int vector, const MhSynArgs* args, int n_m, void* st
   if (nct != 1 && (nct != 2 || a.prec != 1 || !vector)) return MH_EINVAL;
   const int waves = a.waves == 0 ? kSynWavesDefault : a.waves;
   if (waves != 4 && waves != 6) return MH_EINVAL;
+  if (a.prec == 0) return leg_synth_f64(vector, a, n_m, mh_stream(stream));
   const long units =
       (long)mh_cdiv(a.ngroups * a.B, 8 * nct) * mh_cdiv(a.H, 16 * waves) * mh_cdiv(n_m, 8) * 8;
   if (units > 0x7fffffffL) return MH_EINVAL;
   dim3 grid((unsigned)units);
   const dim3 blk(64 * waves);
   hipStream_t st = mh_stream(stream);
-#define MH_SYN_LAUNCH(W)                                                                       \
-  if (nct == 2) {                                                                              \
-    if (a.fprec == 0) hipLaunchKernelGGL((k_syn<true, float, 2, double, W>), grid, blk, 0, st, a, n_m); \
-    else hipLaunchKernelGGL((k_syn<true, float, 2, float, W>), grid, blk, 0, st, a, n_m);       \
-  } else if (a.prec == 0) {                                                                    \
-    if (vector) hipLaunchKernelGGL((k_syn<true, double, 1, double, W>), grid, blk, 0, st, a, n_m); \
-    else hipLaunchKernelGGL((k_syn<false, double, 1, double, W>), grid, blk, 0, st, a, n_m);   \
-  } else if (a.fprec == 0) {                                                                   \
-    if (vector) hipLaunchKernelGGL((k_syn<true, float, 1, double, W>), grid, blk, 0, st, a, n_m); \
-    else hipLaunchKernelGGL((k_syn<false, float, 1, double, W>), grid, blk, 0, st, a, n_m);    \
-  } else {                                                                                     \
-    if (vector) hipLaunchKernelGGL((k_syn<true, float, 1, float, W>), grid, blk, 0, st, a, n_m); \
-    else hipLaunchKernelGGL((k_syn<false, float, 1, float, W>), grid, blk, 0, st, a, n_m);     \
+#define MH_SYN_LAUNCH(W)                                                                     \
+  if (nct == 2) {                                                                            \
+    if (a.fprec == 0) hipLaunchKernelGGL((k_syn<true, 2, double, W>), grid, blk, 0, st, a, n_m); \
+    else hipLaunchKernelGGL((k_syn<true, 2, float, W>), grid, blk, 0, st, a, n_m);           \
+  } else if (a.fprec == 0) {                                                                 \
+    if (vector) hipLaunchKernelGGL((k_syn<true, 1, double, W>), grid, blk, 0, st, a, n_m);   \
+    else hipLaunchKernelGGL((k_syn<false, 1, double, W>), grid, blk, 0, st, a, n_m);         \
+  } else {                                                                                   \
+    if (vector) hipLaunchKernelGGL((k_syn<true, 1, float, W>), grid, blk, 0, st, a, n_m);    \
+    else hipLaunchKernelGGL((k_syn<false, 1, float, W>), grid, blk, 0, st, a, n_m);          \
   }
   if (waves == 4) {
     MH_SYN_LAUNCH(4)
@@ -391,11 +369,11 @@ extern "C" int mh_leg_synth(int vector, const MhSynArgs* args, int n_m, void* st
 // the tile list passed in must have tiles of 16 * waves degrees.
 constexpr int kAnaWavesDefault = 6;
 
-template <bool VEC, typename T, typename FT, int WAVES>
+template <bool VEC, typename FT, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, 2) void k_ana(AnaArgs a, int n_m) {
   const FT* const Fi = reinterpret_cast<const FT*>(a.F);  // Fourier buffer elements
-  typedef Mfma<T> MF;
-  typedef typename MF::acc_t acc_t;
+  typedef float T;
+  typedef float4_t acc_t;
   constexpr int NF = VEC ? 4 : 1;          // f1 same, f1 opposite, f2 same, f2 opposite
   constexpr int NT = 64 * WAVES;
   __shared__ T fs[2][NF][kChunk][16];
@@ -498,15 +476,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_ana(AnaArgs a, int n_m) {
       const int jr = 4 * s + kk;
       const T x1 = fs[buf][0][jr][col];
       if (!VEC) {
-        acc[0] = MF::run(aw, x1, acc[0]);
+        acc[0] = mfma_f32(aw, x1, acc[0]);
       } else {
         const T x2 = fs[buf][1][jr][col];
         const T x3 = fs[buf][2][jr][col];
         const T x4 = fs[buf][3][jr][col];
-        acc[0] = MF::run(ad, x4, acc[0]);  // wdP f2 (opposite fold)
-        acc[1] = MF::run(ad, x2, acc[1]);  // wdP f1 (opposite fold)
-        acc[2] = MF::run(aw, x1, acc[2]);  // wP f1 (same fold)
-        acc[3] = MF::run(aw, x3, acc[3]);  // wP f2 (same fold)
+        acc[0] = mfma_f32(ad, x4, acc[0]);  // wdP f2 (opposite fold)
+        acc[1] = mfma_f32(ad, x2, acc[1]);  // wdP f1 (opposite fold)
+        acc[2] = mfma_f32(aw, x1, acc[2]);  // wP f1 (same fold)
+        acc[3] = mfma_f32(aw, x3, acc[3]);  // wP f2 (same fold)
       }
       const long tn = (long)min(t + D, nsteps - 1) * tstep;
       rW[s % D] = pW[tn];
@@ -539,7 +517,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_ana(AnaArgs a, int n_m) {
   const int bl = bval ? b : 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int k = kbase + MF::row(lane, i);
+    const int k = kbase + mfma_row_f32(lane, i);
     const int l = mo + p + 2 * k;
     const bool st = bval && (k < K);
     const long off = (lms + p + 2 * k) * 2L * a.ldo + 2 * bl + reim;
@@ -572,16 +550,14 @@ extern "C" int mh_leg_analysis(int vector, const MhAnaArgs* args, void* stream) 
   if (a.fprec != 0 && (a.fprec != 1 || a.prec < 1)) return MH_EINVAL;
   hipStream_t st = mh_stream(stream);
   if (a.prec >= 2) return leg_analysis_bf16(vector, a, st);
-#define MH_ANA_LAUNCH(W)                                                                      \
-  if (a.prec == 0) {                                                                          \
-    if (vector) hipLaunchKernelGGL((k_ana<true, double, double, W>), grid, blk, 0, st, a, n_m); \
-    else hipLaunchKernelGGL((k_ana<false, double, double, W>), grid, blk, 0, st, a, n_m);     \
-  } else if (a.fprec == 0) {                                                                  \
-    if (vector) hipLaunchKernelGGL((k_ana<true, float, double, W>), grid, blk, 0, st, a, n_m); \
-    else hipLaunchKernelGGL((k_ana<false, float, double, W>), grid, blk, 0, st, a, n_m);      \
-  } else {                                                                                    \
-    if (vector) hipLaunchKernelGGL((k_ana<true, float, float, W>), grid, blk, 0, st, a, n_m); \
-    else hipLaunchKernelGGL((k_ana<false, float, float, W>), grid, blk, 0, st, a, n_m);       \
+  if (a.prec == 0) return leg_analysis_f64(vector, a, st);
+#define MH_ANA_LAUNCH(W)                                                                    \
+  if (a.fprec == 0) {                                                                       \
+    if (vector) hipLaunchKernelGGL((k_ana<true, double, W>), grid, blk, 0, st, a, n_m);     \
+    else hipLaunchKernelGGL((k_ana<false, double, W>), grid, blk, 0, st, a, n_m);           \
+  } else {                                                                                  \
+    if (vector) hipLaunchKernelGGL((k_ana<true, float, W>), grid, blk, 0, st, a, n_m);      \
+    else hipLaunchKernelGGL((k_ana<false, float, W>), grid, blk, 0, st, a, n_m);            \
   }
   if (waves == 6) {
     MH_ANA_LAUNCH(6)

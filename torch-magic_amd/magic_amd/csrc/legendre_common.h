@@ -1,5 +1,5 @@
-// Helpers shared by the Legendre kernels (legendre.hip: FP64 and FP32 MFMA;
-// legendre_bf16.hip: BF16 split-precision MFMA).
+// Helpers shared by the Legendre kernels (legendre_f64.hip: FP64 MFMA; legendre.hip:
+// FP32 MFMA; legendre_bf16.hip: BF16 split-precision MFMA).
 #pragma once
 
 #include "common.h"
@@ -32,6 +32,9 @@ __device__ __forceinline__ SynIn syn_in(const SynArgs& a, int g, int c) {
 }
 
 
+// FP64 launchers (legendre_f64.hip), for prec 0.
+int leg_synth_f64(int vector, const SynArgs& a, int n_m, hipStream_t st);
+int leg_analysis_f64(int vector, const AnaArgs& a, hipStream_t st);
 // BF16 split-precision launchers (legendre_bf16.hip), for prec 2 and 3.
 int leg_synth_bf16(int vector, const SynArgs& a, int n_m, hipStream_t st);
 int leg_analysis_bf16(int vector, const AnaArgs& a, hipStream_t st);

@@ -61,10 +61,11 @@ class Resolution:
         self.d["l"] = up(self.maps["l"], I32)
         self.d["m"] = up(self.maps["m"], I32)
         self.d["l_rows"] = up(self.maps["l_rows"], I32)
-        for w in (6, 4):
+        for w in (6, 4, "f64"):
             self.d[f"ana_tiles_{w}"] = up(self.lay[f"ana_tiles_{w}"], I32)
         for k, v in self.lmc.items():
             self.d[k] = up(v)
+        self.d["lcf"] = up(self.lay["lcf"])
         for k in ("or1", "or2", "or3", "or4", "r2", "rgrav", "q", "valri2", "valhi2"):
             self.d[k] = up(self.rad[k])
         self.d["ost2_grid"] = up(self.th["ost2_grid"])
@@ -166,7 +167,7 @@ class Resolution:
         BF16 split tables and inputs of that many planes on the BF16 MFMA, FP32
         accumulation.  waves: waves per workgroup (0: the library default; 4 or
         6, 4 only for BF16); nct: column tiles per workgroup (0/1, or 2 for the
-        FP32 and BF16 vector synthesis); same results."""
+        FP32 and BF16 vector synthesis); FP64 chooses its own shape; same results."""
         a = _lib.SynArgs()
         for g, grp in enumerate(groups):
             for c, (x1, x2, mode) in enumerate(grp):
@@ -185,6 +186,7 @@ class Resolution:
         a.Bout = Bout
         a.waves, a.nct = int(waves), int(nct)
         a.minc = self.p.minc
+        a.lcf, a.l_max = ptr(self.d["lcf"]), self.p.l_max
         _lib.call("mh_leg_synth", 1 if vector else 0, _lib.ref(a), self.M, stream_handle())
 
     def analysis(self, F, Bin, B, comps, outS, outT, ldo, vector: bool, prec=0, waves=0):
@@ -192,7 +194,8 @@ class Resolution:
 
         comps: scalar -> list of component indices; vector -> list of (c_vtheta, c_vphi).
         outS/outT: output tensors (or pointers as ints) per component / pair.
-        waves: waves per workgroup (0: the library default, 6; or 4), same results.
+        waves: waves per workgroup (0: the library default, 6; or 4; FP64 has its own
+        work split), same results.
         """
         a = _lib.AnaArgs()
         a.F = ptr(F)
@@ -212,10 +215,11 @@ class Resolution:
         tab, a.mp16 = self._tables(prec)
         a.anaW, a.anaWd = ptr(tab["anaW"]), ptr(tab["anaWd"])
         a.prec = prec
-        w = waves or (4 if prec >= 2 else 6)
+        w = "f64" if prec == 0 else waves or (4 if prec >= 2 else 6)
         a.tiles, a.ntiles = ptr(self.d[f"ana_tiles_{w}"]), self.lay[f"n_ana_tiles_{w}"]
-        a.waves = w
+        a.waves = 0 if prec == 0 else w
         a.n_m, a.minc = self.M, self.p.minc
+        a.lcf, a.l_max = ptr(self.d["lcf"]), self.p.l_max
         _lib.call("mh_leg_analysis", 1 if vector else 0, _lib.ref(a), stream_handle())
 
     def fft(self, forward: bool, F, FB, G, ncomp, B, comp_scale=None):

@@ -216,14 +216,27 @@ def sht_layout(p: Params, maps: dict) -> dict:
         m = mi * p.minc
         for par in range(2):
             K = (p.l_max - m - par) // 2 + 1 if p.l_max - m - par >= 0 else 0
-            K4 = -(-K // 4) * 4
-            K16 = -(-K // 16) * 16
+            Kx = (p.l_max + 1 - m - par) // 2 + 1   # with the degree l_max + 1
+            K4 = -(-Kx // 4) * 4
+            K16 = -(-Kx // 16) * 16
             info[mi, par] = (K, syn_off, ana_off, K16)
             syn_off += K4 * Hp
             ana_off += K16 * Hp
     if syn_off >= 2 ** 31 or ana_off >= 2 ** 31:
         raise ValueError("Legendre tables exceed 32-bit offsets")
-    out = dict(H=H, Hp=Hp, mp_info=info.reshape(-1), syn_size=syn_off, ana_size=ana_off)
+    # the FP64 synthesis reads up to 48 rows past an order's last (and drops them)
+    out = dict(H=H, Hp=Hp, mp_info=info.reshape(-1), syn_size=syn_off + 48 * Hp, ana_size=ana_off)
+    # coupling coefficients of sin(theta) d/dtheta, c_l = sqrt((l^2 - m^2) / (4 l^2 - 1)),
+    # of l = m .. l_max + 1 (one row more per order than the spectral arrays)
+    orders = p.minc * np.arange(p.n_m)
+    l = np.concatenate([np.arange(m, p.l_max + 2) for m in orders]).astype(np.float64)
+    m = np.repeat(orders, p.l_max + 2 - orders).astype(np.float64)
+    c0 = np.sqrt(np.maximum((l - m) * (l + m) / (4.0 * l * l - 1.0), 0.0))
+    c1 = np.sqrt((l + 1.0 - m) * (l + 1.0 + m) / (4.0 * (l + 1.0) ** 2 - 1.0))
+    out["lcf"] = np.stack([(l - 1.0) * c0, (l + 2.0) * c1, (l + 1.0) * c0, l * c1], axis=1)
+    # FP64 analysis: windows of four waves of 15 degree indices
+    win = analysis_windows(p, 60)
+    out["ana_tiles_f64"], out["n_ana_tiles_f64"] = win.reshape(-1), len(win)
     for waves in (6, 4):
         tl = analysis_tiles(p, info, 16 * waves)
         out[f"ana_tiles_{waves}"] = tl.reshape(-1)
@@ -241,6 +254,23 @@ def analysis_tiles(p: Params, info: np.ndarray, tile: int) -> np.ndarray:
         for par in range(2):
             for k0 in range(0, int(info[m, par, 0]), tile):
                 per_xcd[m % 8].append((m, par, k0))
+    return _xcd_lists(p, per_xcd)
+
+
+def analysis_windows(p: Params, window: int) -> np.ndarray:
+    """FP64 analysis work list: one entry per order m and window of degree indices
+    k0 .. (l = m + p + 2 k, both parities), k0 = number * window, as (m, count << 16
+    | number, k0); the window at k0 > 0 writes the degrees from l = m + 2 k0 + 1 on.
+    The windows of an order follow each other.  Lists as analysis_tiles."""
+    per_xcd = [[] for _ in range(8)]
+    for m in range(p.n_m):
+        n = p.l_max + 1 - m * p.minc
+        k0s = [k0 for k0 in range(0, n, window) if k0 == 0 or 2 * k0 + 1 < n]
+        per_xcd[m % 8] += [(m, len(k0s) << 16 | i, k0) for i, k0 in enumerate(k0s)]
+    return _xcd_lists(p, per_xcd)
+
+
+def _xcd_lists(p: Params, per_xcd: list) -> np.ndarray:
     tpx = max(len(t) for t in per_xcd)
     tiles = []
     for t in per_xcd:

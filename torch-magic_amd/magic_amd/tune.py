@@ -125,8 +125,8 @@ def synth_shape(res, N: int, prec: int, fdtype=torch.float64, bufs=None,
     vector (4 groups of N levels) or scalar (one field of N levels), FP64
     (prec 0) or FP32 tables (prec 1) writing Fourier buffers of `fdtype`.
     bufs: (a spectral (L, N) array, the F buffer)."""
-    if os.environ.get("MAGIC_AMD_TUNE", "1") == "0":
-        return (0, 0)
+    if os.environ.get("MAGIC_AMD_TUNE", "1") == "0" or prec == 0:
+        return (0, 0)   # FP64: a rule on the sizes in the library
     fprec = 1 if fdtype == torch.float32 else 0
     ng = 4 if vector else 1
     key = (f"{_device_name(res)}|leg_synth_{'vec' if vector else 'scal'}|L={res.L}|H={res.H}"
@@ -157,8 +157,8 @@ def analysis_waves(res, N: int, prec: int, fdtype=torch.float64, bufs=None) -> i
     dynamo step's), FP64 (prec 0) or FP32 tables (prec 1) reading Fourier
     buffers of `fdtype`.  bufs: (the F buffer of 9 components, an (L, N)
     output array whose boundary columns 0 and N-1 are left untouched)."""
-    if os.environ.get("MAGIC_AMD_TUNE", "1") == "0":
-        return 0
+    if os.environ.get("MAGIC_AMD_TUNE", "1") == "0" or prec == 0:
+        return 0   # FP64 has its own work split
     fprec = 1 if fdtype == torch.float32 else 0
     Nb = N - 2
     key = (f"{_device_name(res)}|leg_analysis_vec|L={res.L}|H={res.H}|M={res.M}|B={Nb}"
