@@ -352,3 +352,48 @@ def test_fp64_transforms_at_tile_edges(l_max, B, minc):
     for a, b in zip(sht.spat_to_sphertor(dev(grids[1]), dev(grids[2])),
                     osht.spat_to_sphertor(grids[1], grids[2])):
         assert np.abs(a.cpu().numpy() - b).max() < tol * np.abs(b).max()
+
+
+@pytest.mark.parametrize("Mh", [2, 3, 5, 12, 24, 30, 45, 48, 64, 96, 128, 150, 192, 225, 288, 300,
+                                384, 500, 576, 648, 720, 768, 800, 1000])
+def test_fft_lengths_match_numpy(Mh):
+    """mh_fft both ways for compiled, run-time and long (> 768) plans, odd and even
+    half lengths, batches that do not fill a workgroup's rows, orders up to Mh;
+    error of a few roundings per pass against numpy."""
+    torch = _torch()
+    from magic_amd import _lib, grid
+    from magic_amd.device import ptr, stream_handle
+    rng = np.random.default_rng(Mh)
+    T, n = 2, 2 * Mh
+    up = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    k = np.arange(Mh)
+    tw, tw2 = np.exp(-2j * np.pi * k / Mh), np.exp(-2j * np.pi * k / n)
+    dtw, dtw2 = up(tw.view(np.float64)), up(tw2.view(np.float64))
+    ost2 = up(np.array([2.0, 3.0]))
+    scale = torch.tensor([0, 1], dtype=torch.int32, device="cuda")
+    for B, M in ((1, max(1, Mh // 3)), (9, Mh), (35, max(1, 2 * Mh // 3))):
+        F = rng.standard_normal((2, M, T, B)) + 1j * rng.standard_normal((2, M, T, B))
+        F[:, 0] = F[:, 0].real
+        full = np.zeros((2, Mh + 1, T, B), complex)
+        full[:, :M] = F
+        g = np.fft.irfft(full, n=n, axis=1, norm="forward").transpose(0, 3, 2, 1)  # (2, B, T, n)
+        dF, dG = up(F), torch.full((2, B, T, n), 7.0, dtype=torch.float64, device="cuda")
+        a = _lib.FftArgs()
+        rad = grid.fft_radices(Mh)
+        a.Mh, a.nstage, a.n_m, a.T, a.B, a.ncomp, a.RB = Mh, len(rad), M, T, B, 2, 1
+        for i, r in enumerate(rad):
+            a.radix[i] = r
+        a.tw, a.tw2, a.ost2 = ptr(dtw), ptr(dtw2), ptr(ost2)
+        a.F, a.Fm_stride, a.Fc_stride, a.FB = ptr(dF), 2 * T * B, 2 * T * B * M, B
+        a.G, a.Gc_stride = ptr(dG), B * T * n
+        tol = 8 * np.finfo(float).eps * np.log2(n)
+        _lib.call("mh_fft", 0, _lib.ref(a), stream_handle())
+        out = dG.cpu().numpy()
+        assert np.abs(out - g).max() < tol * np.abs(g).max(), (B, M)
+        G = rng.standard_normal((2, B, T, n))
+        H = np.fft.rfft(G, axis=3, norm="forward").transpose(0, 3, 2, 1)[:, :M].copy()
+        H[1] *= np.array([2.0, 3.0])[None, :, None]
+        dG.copy_(torch.from_numpy(G))
+        a.comp_scale = ptr(scale)
+        _lib.call("mh_fft", 1, _lib.ref(a), stream_handle())
+        assert np.abs(dF.cpu().numpy() - H).max() < tol * np.abs(H).max(), (B, M)

@@ -52,6 +52,58 @@ __device__ __forceinline__ void dft(V* v, double dir) {
   }
 }
 
+// In-register DFTs of 8 and 9 points (two 4-point / three 3-point DFTs, the
+// constant twiddles, then 2-point / 3-point DFTs).
+template <typename V>
+__device__ __forceinline__ void dft8(V* v, double dir) {
+  typedef decltype(v[0].x) S;
+  const S h = (S)0.70710678118654752440084436210485, d = (S)dir;
+  V a[4] = {v[0], v[2], v[4], v[6]}, b[4] = {v[1], v[3], v[5], v[7]};
+  dft<4>(a, dir);
+  dft<4>(b, dir);
+  // exp(i dir pi q / 4) b_q
+  b[1] = mk2(h * (b[1].x - d * b[1].y), h * (b[1].y + d * b[1].x));
+  b[2] = mk2(-d * b[2].y, d * b[2].x);
+  b[3] = mk2(-h * (b[3].x + d * b[3].y), h * (d * b[3].x - b[3].y));
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    v[q] = cadd(a[q], b[q]);
+    v[q + 4] = csub(a[q], b[q]);
+  }
+}
+
+template <typename V>
+__device__ __forceinline__ void dft9(V* v, double dir) {
+  typedef decltype(v[0].x) S;
+  // exp(i dir 2 pi q / 9), q = 1, 2, 4
+  const V w1 = mk2((S)0.76604444311897803520239265055542, (S)(dir * 0.64278760968653932632264340990726));
+  const V w2 = mk2((S)0.17364817766693034885171662676931, (S)(dir * 0.98480775301220805936674302458952));
+  const V w4 = mk2((S)-0.93969262078590838405410927732473, (S)(dir * 0.34202014332566873304409961468226));
+  V a[3] = {v[0], v[3], v[6]}, b[3] = {v[1], v[4], v[7]}, c[3] = {v[2], v[5], v[8]};
+  dft<3>(a, dir);
+  dft<3>(b, dir);
+  dft<3>(c, dir);
+  b[1] = cmul(b[1], w1);
+  b[2] = cmul(b[2], w2);
+  c[1] = cmul(c[1], w2);
+  c[2] = cmul(c[2], w4);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    V t[3] = {a[q], b[q], c[q]};
+    dft<3>(t, dir);
+    v[q] = t[0];
+    v[q + 3] = t[1];
+    v[q + 6] = t[2];
+  }
+}
+
+template <int R, typename V>
+__device__ __forceinline__ void dft_any(V* v, double dir) {
+  if constexpr (R == 8) dft8(v, dir);
+  else if constexpr (R == 9) dft9(v, dir);
+  else dft<R>(v, dir);
+}
+
 template <int R>
 __device__ void stockham_stage(const double2* __restrict__ in, double2* __restrict__ out, int Mh,
                                int Ns, int RB, const double2* __restrict__ tw, double dir) {
