@@ -23,7 +23,8 @@
 // accumulators and the component being transformed for the force terms),
 // which is why B is transformed twice.
 //
-// FP32 with a compiled plan (the mixed-precision step) runs k_grid_step3, which
+// FP32 with a compiled plan (the mixed-precision step), and FP64 where rows are short,
+// run k_grid_step3, which
 // transforms the three components of each vector together (3*RB LDS rows per
 // pass, a third of the workgroup barriers), with the same arithmetic per value.
 //
@@ -39,14 +40,14 @@ __global__ void k_zero_cfl(unsigned long long* p, int n) {
   if (i < n) p[i] = 0ull;
 }
 
-template <typename T>
+template <int MH, typename T>
 static void launch_generic(const GridArgs& a, const GPlan& P, dim3 gd, dim3 bd, size_t lds,
                            hipStream_t st) {
   switch (P.RL) {
-    case 2: hipLaunchKernelGGL((k_grid_step<0, 2, T, 0>), gd, bd, lds, st, a, P); break;
-    case 3: hipLaunchKernelGGL((k_grid_step<0, 3, T, 0>), gd, bd, lds, st, a, P); break;
-    case 4: hipLaunchKernelGGL((k_grid_step<0, 4, T, 0>), gd, bd, lds, st, a, P); break;
-    default: hipLaunchKernelGGL((k_grid_step<0, 5, T, 0>), gd, bd, lds, st, a, P); break;
+    case 2: hipLaunchKernelGGL((k_grid_step<MH, 2, T, 0>), gd, bd, lds, st, a, P); break;
+    case 3: hipLaunchKernelGGL((k_grid_step<MH, 3, T, 0>), gd, bd, lds, st, a, P); break;
+    case 4: hipLaunchKernelGGL((k_grid_step<MH, 4, T, 0>), gd, bd, lds, st, a, P); break;
+    default: hipLaunchKernelGGL((k_grid_step<MH, 5, T, 0>), gd, bd, lds, st, a, P); break;
   }
 }
 
@@ -59,22 +60,11 @@ extern "C" int mh_grid_plan(int Mh, int* out) {
   return MH_OK;
 }
 
-// Whether Mh has a compiled plan (the FP32 launch of a compiled plan
-// transforms three components together and needs three times the LDS rows).
-static bool grid_compiled(int Mh) {
-  switch (Mh) {
-#define MH_CCASE(V) case V:
-    MH_GRID_COMPILED(MH_CCASE)
-#undef MH_CCASE
-    return true;
-    default: return false;
-  }
-}
-
 extern "C" int mh_grid_step(const MhGridArgs* args, void* stream) {
   const GridArgs& a = *args;
   if (a.N < 3 || a.T < 1 || a.Mh < 2 || a.M < 1 || a.M > a.Mh) return MH_EINVAL;
-  GPlan P = make_plan(a.Mh);
+  const bool wide = wide_plan(a.Mh, a.fprec == 1 ? 4 : 8);
+  GPlan P = make_plan(a.Mh, wide);
   if (P.RL == 0) return MH_EINVAL;
   // level block: the plan's own (the most levels that fit), or a.rb fewer
   const int own_rb = P.RB;
@@ -82,7 +72,7 @@ extern "C" int mh_grid_step(const MhGridArgs* args, void* stream) {
   const int rb = a.rb > 0 ? a.rb : own_rb;
   P.RB = rb;
   P.threads = (rb * P.TP + 63) / 64 * 64;
-  if (rb == own_rb) P.threads = make_plan(a.Mh).threads;
+  if (rb == own_rb) P.threads = make_plan(a.Mh, wide).threads;
   // every thread covers its share of the (Mh/2 + 1) * RB conjugate-pair items
   if (a.Mh % 2 != 0 || (long)P.threads * ((P.RL + 2) / 2) < (long)(a.Mh / 2 + 1) * P.RB)
     return MH_EINVAL;
@@ -93,9 +83,13 @@ extern "C" int mh_grid_step(const MhGridArgs* args, void* stream) {
   if ((long)a.T * 4 * a.N * 2 >= (1L << 24) || (long)a.M * a.T * 4 * a.N * 2 >= (1L << 31))
     return MH_EINVAL;
   const size_t esz = a.fprec ? sizeof(float2) : sizeof(double2);
-  const bool batched =
-      a.fprec && !a.generic && (rb == own_rb || rb == 1 || rb == 2) && grid_compiled(a.Mh);
-  const size_t lds = (2ull * (batched ? 3 : 1) * P.RB * (a.Mh + 2) + 2ull * a.Mh) * esz;
+  const auto lds_of = [&](int comps) {
+    return (2ull * comps * P.RB * P.LS + 2ull * a.Mh) * esz;
+  };
+  const bool compiled = !a.generic && (rb == own_rb || rb == 1 || rb == 2) && grid_compiled(a.Mh);
+  const bool batched = compiled && grid_batched(a.Mh, rb == own_rb ? 0 : rb, a.fprec ? 4 : 8) &&
+                       lds_of(3) <= (size_t)kLdsBytes;
+  const size_t lds = lds_of(batched ? 3 : 1);
   if (lds > (size_t)kLdsBytes) return MH_EINVAL;
   const int nRB = (a.N + P.RB - 1) / P.RB;
   const long nwg = (long)a.T * nRB;
@@ -106,7 +100,8 @@ extern "C" int mh_grid_step(const MhGridArgs* args, void* stream) {
   const dim3 gd((unsigned)grid), bd(P.threads);
   hipStream_t st = mh_stream(stream);
   bool done = false;
-  if (!a.generic) {
+  // compiled kernels: batched, or the FP64 ones that are never batched
+  if (compiled && (batched || !grid_batched(a.Mh, rb == own_rb ? 0 : rb, a.fprec ? 4 : 8))) {
     if (rb == own_rb)
       done = a.fprec ? launch_compiled<0, float>(a, P, gd, bd, lds, st)
                      : launch_compiled<0, double>(a, P, gd, bd, lds, st);
@@ -116,8 +111,10 @@ extern "C" int mh_grid_step(const MhGridArgs* args, void* stream) {
       done = grid_launch_rb2(a, P, gd, bd, lds, st);
   }
   if (!done) {
-    if (a.fprec) launch_generic<float>(a, P, gd, bd, lds, st);
-    else launch_generic<double>(a, P, gd, bd, lds, st);
+    if (a.fprec && P.pad) launch_generic<-1, float>(a, P, gd, bd, lds, st);
+    else if (a.fprec) launch_generic<0, float>(a, P, gd, bd, lds, st);
+    else if (P.pad) launch_generic<-1, double>(a, P, gd, bd, lds, st);
+    else launch_generic<0, double>(a, P, gd, bd, lds, st);
   }
   return mh_launch_status();
 }

@@ -15,20 +15,67 @@ constexpr int kLdsBytes = 160 * 1024 - 256;
 
 // FFT plan of the fused kernel for a half length Mh: radices in inverse order,
 // the last (RL) being the register pass; TP = Mh/RL threads per level; RB
-// levels per workgroup.  LDS: two buffers of RB rows of Mh+1 complex values,
-// then the twiddles exp(-2 pi i k/Mh) and exp(-2 pi i k/(2Mh)), k < Mh.  Rows
-// are Mh+2 values long (even, so every row starts on 16 bytes in FP32).
+// levels per workgroup.  LDS: two buffers of RB rows of LS complex values,
+// then the twiddles exp(-2 pi i k/Mh) and exp(-2 pi i k/(2Mh)), k < Mh.
+//
+// Two kinds of LDS passes (wide_plan() chooses): radix 4, or (`wide`) radix 8 with
+// odd radices first, one pass, one barrier and a fifth of the LDS traffic less
+// (Mh = 576: 3, 8, 8 and the register radix 3, against 4, 4, 4, 3).  Wide passes, and
+// the passes behind an odd radix, pad: a pass writes groups of Ns*R elements, and one
+// element of padding after each group keeps lanes that write the same place of
+// consecutive groups on different banks; it costs the next pass nothing, whose Ns is
+// the group, so that element bf + r*nb sits at bf + bf/Ns + r*(nb + nb/Ns).
 struct GPlan {
   int RL, TP, RB, nst, threads;
   int radix[16];
+  int LS;  // LDS row length
+  bool pad;
+  // ceil(2^32 / d) of the run-time plan's divisors, x / d = umulhi(x, m) for x < 2^16:
+  // butterflies per row of each pass, and its Ns in the inverse and forward order
+  unsigned mnb[16], mni[16], mnf[16];
 };
 
-constexpr GPlan make_plan(int Mh) {
+// Whether a padding plan pads groups of `group` elements: even groups of 8 to 32 (an
+// odd group length spreads by itself, a long one is contiguous for whole waves,
+// and one element in four would be too much LDS).
+constexpr bool pads(int group) { return group % 2 == 0 && group >= 8 && group <= 32; }
+
+// Half lengths with a compiled plan (all divisions and stage loops resolved
+// at compile time); other lengths run the same code with the run-time plan.
+#define MH_GRID_COMPILED(X) \
+  X(24) X(48) X(64) X(72) X(96) X(128) X(144) X(192) X(256) X(288) X(384) X(576) X(768)
+constexpr bool grid_compiled(int Mh) {
+  switch (Mh) {
+#define MH_CCASE(V) case V:
+    MH_GRID_COMPILED(MH_CCASE)
+#undef MH_CCASE
+    return true;
+    default: return false;
+  }
+}
+
+// Kind of plan, by length and element size only, so that every level block, batched
+// or not, compiled or not, gives the same results bit for bit.  Wide where three
+// components are transformed together in workgroups of some waves: their 9/8
+// butterflies per thread cost a second round to one wave in eight (FP32, l_max = 383,
+// 97 levels: 2.77 -> 2.38 ms; l_max = 85, FP64: 114 -> 108 us); in one or two waves the
+// second round is the whole pass again (l_max = 64, FP32: 50 against 55 us), and a
+// single component of one level (long FP64 rows) has 72 butterflies for 192 threads
+// (l_max = 383: 4.34 against 4.72 ms).
+constexpr bool wide_plan(int Mh, int esz) {
+  return grid_compiled(Mh) && Mh >= 128 && (esz == 4 || Mh <= 128);
+}
+
+constexpr GPlan make_plan(int Mh, bool wide = false) {
   GPlan p{};
   if (Mh < 2) return p;
   const int RL = Mh % 3 == 0 ? 3 : Mh % 4 == 0 ? 4 : Mh % 2 == 0 ? 2 : Mh % 5 == 0 ? 5 : 0;
   if (RL == 0) return p;
   int n = Mh / RL, k = 0;
+  // odd radices first in padding plans: their first pass writes at an odd stride
+  p.pad = wide || (grid_compiled(Mh) && n % 3 == 0);
+  while (p.pad && n % 3 == 0 && k < 15) { p.radix[k++] = 3; n /= 3; }
+  while (wide && n % 8 == 0 && k < 15) { p.radix[k++] = 8; n /= 8; }
   while (n % 4 == 0 && k < 15) { p.radix[k++] = 4; n /= 4; }
   while (n % 2 == 0 && k < 15) { p.radix[k++] = 2; n /= 2; }
   while (n % 3 == 0 && k < 15) { p.radix[k++] = 3; n /= 3; }
@@ -37,9 +84,26 @@ constexpr GPlan make_plan(int Mh) {
   p.radix[k++] = RL;
   p.nst = k;
   p.TP = Mh / RL;
+  // the longest padding of either direction's passes (even: rows start on 16 bytes)
+  p.LS = Mh + 2;
+  for (int s = 0, up = 1, dn = 1; s < k; ++s) {
+    up *= p.radix[s];
+    dn *= p.radix[k - 1 - s];
+    if (p.pad && pads(up) && Mh + Mh / up + 2 > p.LS) p.LS = Mh + Mh / up + 2;
+    if (p.pad && pads(dn) && Mh + Mh / dn + 2 > p.LS) p.LS = Mh + Mh / dn + 2;
+  }
+  p.LS += p.LS % 2;
+  for (int s = 0, up = 1, dn = 1; s < k; ++s) {
+    const int f = k - 1 - s;
+    p.mnb[s] = (unsigned)(((1ull << 32) + Mh / p.radix[s] - 1) / (Mh / p.radix[s]));
+    p.mni[s] = up > 1 ? (unsigned)(((1ull << 32) + up - 1) / up) : 0u;
+    p.mnf[f] = dn > 1 ? (unsigned)(((1ull << 32) + dn - 1) / dn) : 0u;
+    up *= p.radix[s];
+    dn *= p.radix[f];
+  }
   for (int rb = 16; rb >= 1; --rb) {
     const int th = (rb * p.TP + 63) / 64 * 64;
-    if (th <= kMaxThreads && (2 * rb * (Mh + 2) + 2 * Mh) * 16 <= kLdsBytes) {
+    if (th <= kMaxThreads && (2 * rb * p.LS + 2 * Mh) * 16 <= kLdsBytes) {
       p.RB = rb;
       p.threads = th;
       break;
@@ -49,10 +113,6 @@ constexpr GPlan make_plan(int Mh) {
   return p;
 }
 
-// Half lengths with a compiled plan (all divisions and stage loops resolved
-// at compile time); other lengths run the same code with the run-time plan.
-#define MH_GRID_COMPILED(X) X(24) X(48) X(96) X(192) X(288) X(384) X(576) X(768)
-
 // Workgroup barrier that waits for this wave's LDS operations only, so the
 // global loads of the next component stay in flight across FFT passes.
 __device__ __forceinline__ void lds_barrier() {
@@ -61,36 +121,41 @@ __device__ __forceinline__ void lds_barrier() {
 
 extern __shared__ double2 g_lds_raw[];
 
-// Geometry of one launch; compile-time constants when MH > 0.
+// Geometry of one launch; compile-time constants when MH > 0.  MH = 0 runs a run-time
+// plan without radix 8 and padding, MH = -1 one with them.
 struct Geo {
   int Mh, M, RB, LS, TP, nst, threads;
+  bool pad;
   int RBL;  // rows per LDS buffer: RB levels times the components transformed together
 };
 
-template <int MH, int RBC, int NB = 1>
+template <int MH, int RBC, typename T, int NB = 1>
 __device__ __forceinline__ Geo make_geo(const GridArgs& a, const GPlan& rp) {
   Geo g;
   g.M = a.M;
   if constexpr (MH > 0) {
-    constexpr GPlan P = make_plan(MH);
+    constexpr GPlan P = make_plan(MH, wide_plan(MH, sizeof(T)));
     g.Mh = MH;
     g.RB = RBC > 0 ? RBC : P.RB;
     g.TP = P.TP;
     g.nst = P.nst;
+    g.LS = P.LS;
+    g.pad = P.pad;
     g.threads = RBC > 0 ? (RBC * P.TP + 63) / 64 * 64 : P.threads;
   } else {
     g.Mh = a.Mh;
     g.RB = rp.RB;
     g.TP = rp.TP;
     g.nst = rp.nst;
+    g.LS = rp.LS;
+    g.pad = MH < 0 && rp.pad;
     g.threads = rp.threads;
   }
-  g.LS = g.Mh + 2;
   g.RBL = g.RB * NB;
   return g;
 }
 
-// LDS: two buffers of RB rows of Mh+1 complex values, then the twiddles, all
+// LDS: two buffers of RB rows of LS complex values, then the twiddles, all
 // in the element type of the launch
 template <typename T>
 __device__ __forceinline__ typename vec2<T>::type* lds_base() {
@@ -116,35 +181,57 @@ struct Ctx {
   int busy;         // LDS buffer that other threads may still be reading
 };
 
-template <int R, typename T>
+// One LDS pass of radix R.  Input groups (Ns) and output groups (Ns*R) are padded
+// by the rule of pads() (a group of one, the packed spectrum, has none).
+template <int R, typename T, bool PAD>
 __device__ __forceinline__ void stage_mid(const Geo& g, const GridArgs& a, int win, int wout, int Ns,
-                                          double dir, int nrows) {
+                                          double dir, int nrows, unsigned mnb = 0, unsigned mns = 0) {
   typedef typename vec2<T>::type V;
   const int nb = g.Mh / R, tstep = g.Mh / (Ns * R);
+  const bool pin = PAD && pads(Ns), pout = PAD && pads(Ns * R);
+  const int rstep = pin ? nb + nb / Ns : nb, gstep = Ns * R + (pout ? 1 : 0);
   const V* tw = ltw<T>(g);
   const V* in = lbuf<T>(g, win);
   V* out = lbuf<T>(g, wout);
   for (int idx = threadIdx.x; idx < nrows * nb; idx += g.threads) {
-    const int row = idx / nb, bf = idx - row * nb;
-    const int k = bf % Ns;
-    const V* src = in + row * g.LS;
+    // run-time divisors by their reciprocals (a division takes some 25 instructions)
+    const int row = mnb ? (int)__umulhi((unsigned)idx, mnb) : idx / nb, bf = idx - row * nb;
+    const int gr = Ns == 1 ? bf : mns ? (int)__umulhi((unsigned)bf, mns) : bf / Ns, k = bf - gr * Ns;
+    const V* src = in + row * g.LS + bf + (pin ? gr : 0);
     V v[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = src[bf + r * nb];
+    for (int r = 0; r < R; ++r) v[r] = src[r * rstep];
     if (Ns > 1) {
-      // w^r by recurrence from one table value (one LDS read per butterfly)
-      V w1 = tw[k * tstep];
-      w1.y *= (T)-dir;  // tw holds exp(-i...); the inverse (dir = +1) conjugates
-      V wr = w1;
+      // powers of w by products from one table value (exp(-i...); the inverse
+      // conjugates), for radix 8 from w and w^2, so that none is more than
+      // three products deep
+      auto get = [&](int r) {
+        V w = tw[r * k * tstep];
+        w.y *= (T)-dir;
+        return w;
+      };
+      const V w1 = get(1);
+      if constexpr (R == 8) {
+        const V w2 = get(2), w3 = cmul(w1, w2), w4 = cmul(w2, w2);
+        v[1] = cmul(v[1], w1);
+        v[2] = cmul(v[2], w2);
+        v[3] = cmul(v[3], w3);
+        v[4] = cmul(v[4], w4);
+        v[5] = cmul(v[5], cmul(w1, w4));
+        v[6] = cmul(v[6], cmul(w2, w4));
+        v[7] = cmul(v[7], cmul(w3, w4));
+      } else {
+        V wr = w1;
 #pragma unroll
-      for (int r = 1; r < R; ++r) {
-        v[r] = cmul(v[r], wr);
-        if (r + 1 < R) wr = cmul(wr, w1);
+        for (int r = 1; r < R; ++r) {
+          v[r] = cmul(v[r], wr);
+          if (r + 1 < R) wr = cmul(wr, w1);
+        }
       }
     }
-    dft<R>(v, dir);
-    V* dst = out + row * g.LS + (bf / Ns) * Ns * R + k;
-    if constexpr (sizeof(T) == 4 && R % 2 == 0) {
+    dft_any<R>(v, dir);
+    V* dst = out + row * g.LS + gr * gstep + k;
+    if constexpr (sizeof(T) == 4 && R == 4) {
       if (Ns == 1) {
         // consecutive outputs from an even element: 16-byte stores of pairs
         // (half the store instructions at this pass's stride of R values)
@@ -159,22 +246,27 @@ __device__ __forceinline__ void stage_mid(const Geo& g, const GridArgs& a, int w
   }
 }
 
-template <typename T>
+// Run-time radix; radix 8 and padding only where WIDE: its registers would spill in
+// the kernels that never use it.
+template <typename T, bool WIDE>
 __device__ __forceinline__ void stage_mid_rt(const Geo& g, const GridArgs& a, int R, int win, int wout,
-                                             int Ns, double dir, int nrows) {
-  if (R == 4) stage_mid<4, T>(g, a, win, wout, Ns, dir, nrows);
-  else if (R == 2) stage_mid<2, T>(g, a, win, wout, Ns, dir, nrows);
-  else if (R == 3) stage_mid<3, T>(g, a, win, wout, Ns, dir, nrows);
-  else stage_mid<5, T>(g, a, win, wout, Ns, dir, nrows);
+                                             int Ns, double dir, int nrows, unsigned mnb,
+                                             unsigned mns) {
+  if (WIDE && R == 8) {
+    if constexpr (WIDE) stage_mid<8, T, WIDE>(g, a, win, wout, Ns, dir, nrows, mnb, mns);
+  } else if (R == 4) stage_mid<4, T, WIDE>(g, a, win, wout, Ns, dir, nrows, mnb, mns);
+  else if (R == 2) stage_mid<2, T, WIDE>(g, a, win, wout, Ns, dir, nrows, mnb, mns);
+  else if (R == 3) stage_mid<3, T, WIDE>(g, a, win, wout, Ns, dir, nrows, mnb, mns);
+  else stage_mid<5, T, WIDE>(g, a, win, wout, Ns, dir, nrows, mnb, mns);
 }
 
 // Inverse stages 0 .. nst-2 of a compiled plan (S = stage, NS = its Ns).
 template <int MH, int S, int NS, typename T>
 __device__ __forceinline__ int inv_mid_ct(const Geo& g, const GridArgs& a, int w, int nrows) {
-  constexpr GPlan P = make_plan(MH);
+  constexpr GPlan P = make_plan(MH, wide_plan(MH, sizeof(T)));
   if constexpr (S < P.nst - 1) {
     constexpr int R = P.radix[S];
-    stage_mid<R, T>(g, a, w, 1 - w, NS, 1.0, nrows);
+    stage_mid<R, T, P.pad>(g, a, w, 1 - w, NS, 1.0, nrows);
     lds_barrier();
     return inv_mid_ct<MH, S + 1, NS * R, T>(g, a, 1 - w, nrows);
   } else {
@@ -185,10 +277,10 @@ __device__ __forceinline__ int inv_mid_ct(const Geo& g, const GridArgs& a, int w
 // Forward stages S = nst-2 .. 0 of a compiled plan.
 template <int MH, int S, int NS, typename T>
 __device__ __forceinline__ int fwd_mid_ct(const Geo& g, const GridArgs& a, int w, int nrows) {
-  constexpr GPlan P = make_plan(MH);
+  constexpr GPlan P = make_plan(MH, wide_plan(MH, sizeof(T)));
   if constexpr (S >= 0) {
     constexpr int R = P.radix[S];
-    stage_mid<R, T>(g, a, w, 1 - w, NS, -1.0, nrows);
+    stage_mid<R, T, P.pad>(g, a, w, 1 - w, NS, -1.0, nrows);
     lds_barrier();
     return fwd_mid_ct<MH, S - 1, NS * R, T>(g, a, 1 - w, nrows);
   } else {
@@ -233,6 +325,15 @@ __device__ __forceinline__ void fetch(const Geo& g, const GridArgs& a, Prefetch<
       if (p > 0 && 2 * p < g.Mh) pf.xc[i] = ld(g.Mh - p, j);
     }
   }
+}
+
+// Whether a compiled plan transforms three components together: always in FP32; in
+// FP64 for short rows with one or two levels per workgroup, where barriers bound the
+// passes (two levels: l_max = 16, 33 levels 27 -> 20 us; l_max = 64, 65 levels 100 -> 85
+// us), while long rows lose more workgroups per CU to the LDS and registers of three
+// than the barriers cost (l_max = 383, 97 levels: 5.5 ms against 4.3 one by one).
+constexpr bool grid_batched(int Mh, int rbc, int esz) {
+  return esz == 4 || (Mh <= 128 && (rbc == 1 || rbc == 2));
 }
 
 struct NoFetch {
@@ -282,7 +383,8 @@ __device__ __forceinline__ void inverse(Ctx& c, const Geo& g, const GridArgs& a,
       const GPlan& P = *c.rp;
       int Ns = 1;
       for (int s = 0; s < P.nst - 1; ++s) {
-        stage_mid_rt<T>(g, a, P.radix[s], w, 1 - w, Ns, 1.0, g.RB);
+        stage_mid_rt<T, MH < 0>(g, a, P.radix[s], w, 1 - w, Ns, 1.0, g.RB,
+                                     P.mnb[s], P.mni[s]);
         Ns *= P.radix[s];
         w = 1 - w;
         lds_barrier();
@@ -294,7 +396,7 @@ __device__ __forceinline__ void inverse(Ctx& c, const Geo& g, const GridArgs& a,
     const V* src = lbuf<T>(g, w) + c.row * LS;
     const V* tw = ltw<T>(g);
 #pragma unroll
-    for (int i = 0; i < RL; ++i) z[i] = src[c.q + i * g.TP];
+    for (int i = 0; i < RL; ++i) z[i] = src[c.q + i * (g.TP + (g.pad && pads(g.TP) ? 1 : 0))];
     if (g.nst > 1) {
       const V w1 = cconj(tw[c.q]);
       V wi = w1;
@@ -330,13 +432,14 @@ __device__ __forceinline__ void forward(Ctx& c, const Geo& g, const GridArgs& a,
   }
   lds_barrier();
   if constexpr (MH > 0) {
-    constexpr GPlan P = make_plan(MH);
+    constexpr GPlan P = make_plan(MH, wide_plan(MH, sizeof(T)));
     w = fwd_mid_ct<MH, P.nst - 2, RL, T>(g, a, w, g.RB);
   } else {
     const GPlan& P = *c.rp;
     int Ns = RL;
     for (int s = P.nst - 2; s >= 0; --s) {
-      stage_mid_rt<T>(g, a, P.radix[s], w, 1 - w, Ns, -1.0, g.RB);
+      stage_mid_rt<T, MH < 0>(g, a, P.radix[s], w, 1 - w, Ns, -1.0, g.RB,
+                                   P.mnb[s], P.mnf[s]);
       Ns *= P.radix[s];
       w = 1 - w;
       lds_barrier();
@@ -460,7 +563,7 @@ __device__ __forceinline__ void inverseN(Ctx& c, const Geo& g, const GridArgs& a
     for (int k = 0; k < NC; ++k) {
       const V* src = lbuf<T>(g, w) + (k * RB + c.row) * LS;
 #pragma unroll
-      for (int i = 0; i < RL; ++i) z[k][i] = src[c.q + i * g.TP];
+      for (int i = 0; i < RL; ++i) z[k][i] = src[c.q + i * (g.TP + (g.pad && pads(g.TP) ? 1 : 0))];
       if (g.nst > 1) {
         V wi = w1;
 #pragma unroll
@@ -500,7 +603,7 @@ __device__ __forceinline__ void forwardN(Ctx& c, const Geo& g, const GridArgs& a
   }
   lds_barrier();
   {
-    constexpr GPlan P = make_plan(MH);
+    constexpr GPlan P = make_plan(MH, wide_plan(MH, sizeof(T)));
     w = fwd_mid_ct<MH, P.nst - 2, RL, T>(g, a, w, NC * RB);
   }
   const int Mh = g.Mh, N = a.N, No = N - 2, n = (Mh / 2 + 1) * RB;
@@ -543,7 +646,7 @@ template <int MH, int RL, typename T, int RBC>
 __global__ __launch_bounds__(kMaxThreads, 3) void k_grid_step(GridArgs a, GPlan rp) {
   typedef typename vec2<T>::type V;
   __shared__ unsigned long long red[2 * 16];
-  const Geo g = make_geo<MH, RBC>(a, rp);
+  const Geo g = make_geo<MH, RBC, T>(a, rp);
   const int N = a.N, nth = a.T, RB = g.RB;
   const int nRB = (N + RB - 1) / RB;
   // XCD-aware order: workgroups i and i+8 are dispatched to the same XCD, so
@@ -758,12 +861,17 @@ __global__ __launch_bounds__(kMaxThreads, 3) void k_grid_step(GridArgs a, GPlan 
 // FP32 grid step of the compiled plans with the vector components transformed
 // together (inverseN / forwardN over 3*RB LDS rows).  Same arithmetic per
 // value as k_grid_step<MH, RL, float, RBC>, in the same order.
-template <int MH, int RL, int RBC>
-__global__ __launch_bounds__(kMaxThreads, 3) void k_grid_step3(GridArgs a, GPlan rp) {
-  typedef float T;
+template <int MH, int RBC>
+constexpr int plan_threads() {
+  return RBC > 0 ? (RBC * make_plan(MH).TP + 63) / 64 * 64 : make_plan(MH).threads;
+}
+
+template <int MH, int RL, typename T, int RBC>
+__global__ __launch_bounds__((plan_threads<MH, RBC>()), (sizeof(T) == 4 ? 3 : 2)) void k_grid_step3(
+    GridArgs a, GPlan rp) {
   typedef typename vec2<T>::type V;
   __shared__ unsigned long long red[2 * 16];
-  const Geo g = make_geo<MH, RBC, 3>(a, rp);
+  const Geo g = make_geo<MH, RBC, T, 3>(a, rp);
   const int N = a.N, nth = a.T, RB = g.RB;
   const int nRB = (N + RB - 1) / RB;
   const int nwg = nth * nRB, per = (nwg + 7) / 8;
@@ -961,8 +1069,8 @@ bool launch_compiled(const GridArgs& a, const GPlan& P, dim3 gd, dim3 bd, size_t
   switch (a.Mh) {
 #define MH_CASE(V)                                                                       \
   case V:                                                                                \
-    if constexpr (sizeof(T) == 4)                                                        \
-      hipLaunchKernelGGL((k_grid_step3<V, make_plan(V).RL, RBC>), gd, bd, lds, st, a, P); \
+    if constexpr (grid_batched(V, RBC, sizeof(T)))                                       \
+      hipLaunchKernelGGL((k_grid_step3<V, make_plan(V).RL, T, RBC>), gd, bd, lds, st, a, P); \
     else                                                                                 \
       hipLaunchKernelGGL((k_grid_step<V, make_plan(V).RL, T, RBC>), gd, bd, lds, st, a, P); \
     return true;
