@@ -397,3 +397,24 @@ def test_fft_lengths_match_numpy(Mh):
         a.comp_scale = ptr(scale)
         _lib.call("mh_fft", 1, _lib.ref(a), stream_handle())
         assert np.abs(dF.cpu().numpy() - H).max() < tol * np.abs(H).max(), (B, M)
+
+
+def test_sphertor_inputs_of_any_layout():
+    """spat_to_sphertor reads the grids in place: a strided view, a view that does
+    not start on 16 bytes and one phi field for a batch of theta fields give the
+    results of plain copies."""
+    torch = _torch()
+    from magic_amd.params import Params
+    from magic_amd.device import Resolution
+    from magic_amd.sht import SHT
+    res = Resolution(Params({"l_max": 16, "n_r_max": 9}))
+    sht = SHT(res)
+    T, P = res.T, res.P
+    base = torch.randn(3 * T * P + 1, dtype=torch.float64, device="cuda")
+    vt = base[1:].view(3, T, P)
+    vp = torch.randn(P, 3, T, dtype=torch.float64, device="cuda").permute(1, 2, 0)
+    ref = sht.spat_to_sphertor(vt.clone(), vp.contiguous().clone())
+    assert all(torch.equal(a, b) for a, b in zip(sht.spat_to_sphertor(vt, vp), ref))
+    one = sht.spat_to_sphertor(vt, vp[:1])
+    full = sht.spat_to_sphertor(vt, vp[:1].expand(3, T, P).contiguous())
+    assert all(torch.equal(a, b) for a, b in zip(one, full))

@@ -43,7 +43,8 @@ def _grid(x, T, P):
     x = x if batched else x.unsqueeze(0)
     if tuple(x.shape[1:]) != (T, P):
         raise ValueError(f"expected grid ({T}, {P}), got {tuple(x.shape[1:])}")
-    return x.contiguous(), batched
+    x = x.contiguous()
+    return (x.clone() if x.data_ptr() % 16 else x), batched   # rows are read in 16-byte pairs
 
 
 class SHT:
@@ -85,7 +86,7 @@ class SHT:
         B = g.shape[0]
         F = r.fourier_buffer(1, B)
         r.fft(True, F, B, g, 1, B)
-        out = torch.zeros(r.L, B, dtype=C128, device=r.device)
+        out = torch.empty(r.L, B, dtype=C128, device=r.device)   # every row is written
         r.analysis(F, B, B, [0], [out], [None], B, vector=False, prec=self.prec)
         return out if batched else out[:, 0]
 
@@ -109,13 +110,14 @@ class SHT:
         t, batched = _grid(vt, r.T, r.P)
         p, _ = _grid(vp, r.T, r.P)
         B = t.shape[0]
-        G = torch.empty(2, B, r.T, r.P, dtype=F64, device=r.device)
-        G[0].copy_(self._on(t))
-        G[1].copy_(self._on(p))
         F = r.fourier_buffer(2, B)
-        r.fft(True, F, B, G, 2, B, comp_scale=r.d["comp_scale_2"])
-        S = torch.zeros(r.L, B, dtype=C128, device=r.device)
-        T = torch.zeros(r.L, B, dtype=C128, device=r.device)
+        half = F.numel() // 2
+        if p.shape[0] != B:   # one field for the whole batch
+            p = p.expand(B, r.T, r.P).contiguous()
+        for c, g in enumerate((self._on(t), self._on(p))):   # from the inputs, without a copy
+            r.fft(True, F[c * half:], B, g, 1, B, comp_scale=r.d["comp_scale_2"])
+        S = torch.empty(r.L, B, dtype=C128, device=r.device)
+        T = torch.empty(r.L, B, dtype=C128, device=r.device)
         r.analysis(F, B, B, [(0, 1)], [S], [T], B, vector=True, prec=self.prec)
         return (S, T) if batched else (S[:, 0], T[:, 0])
 
