@@ -77,6 +77,46 @@ def test_band_factor_pivots_and_solve_config3_sizes(kl, ku, dominant):
         assert np.abs(res).max() < 1e-10 * np.abs(fac[l][None, :] * rhs[rows]).max()
 
 
+@pytest.mark.parametrize("kl,ku,n", [(0, 2, 5), (1, 0, 16), (1, 4, 17), (2, 2, 1), (2, 2, 33), (3, 3, 48),
+                                     (3, 3, 95), (4, 0, 3), (4, 4, 16), (4, 4, 65)])
+@pytest.mark.parametrize("scale", [1.0, 1e290])
+def test_band_solve_tiles_and_degrees_per_wave(kl, ku, n, scale):
+    """Column counts around the 16-column tiles, waves of one to eight and of more
+    degrees (rows in order and not), a ragged last wave, pivots whose reciprocal the
+    kernel does not use (``scale`` 1e290), both scalings, in place and out.
+    Diagonally dominant systems: the condition number is a few tens, so 1e-13 of
+    the largest entry is some 30 roundings times that."""
+    import torch
+    from magic_amd import _lib
+    from magic_amd import algebra as A
+    from magic_amd.device import ptr, stream_handle
+    from oracle import algebra as O
+    rng = np.random.default_rng(100 * n + 10 * kl + ku)
+    nl = 40
+    dense = np.stack([_band(n, kl, ku, rng, True) for _ in range(nl)])
+    dense /= np.abs(np.einsum("lii->li", dense))[:, :, None]
+    abd = np.stack([O.dense_to_band_storage(scale * d, kl, ku) for d in dense])
+    gabd, gpiv, ginfo = A.prepare_band_batched(torch.from_numpy(abd), n, kl, ku)
+    assert not ginfo.any()
+    fr, fc = rng.uniform(0.5, 2.0, (2, nl, n))
+    for lidx in (np.sort(np.concatenate([np.arange(m, nl) for m in range(nl)]))[:803],
+                 rng.integers(0, nl, 70)):
+        rhs = rng.standard_normal((lidx.size, n)) + 1j * rng.standard_normal((lidx.size, n))
+        ref = np.stack([fc[l] * np.linalg.solve(dense[l], fr[l] * b) for l, b in zip(lidx, rhs)])
+        dev = torch.device("cuda")
+        t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(dev)
+        li, r, frd, fcd = t(lidx.astype(np.int32)), t(scale * rhs), t(fr), t(fc)
+        gp = gpiv.to(dev).to(torch.int32).contiguous()
+        order = torch.argsort(li, stable=True).to(torch.int32)
+        for rows in (None, ptr(order)):
+            for inplace in (False, True):
+                src = r.clone()
+                out = src if inplace else torch.empty_like(r)
+                _lib.call("mh_band_solve", ptr(gabd), ptr(gp), ptr(frd), ptr(fcd), ptr(li), rows,
+                          ptr(src), ptr(out), lidx.size, n, kl, ku, stream_handle())
+                assert np.abs(out.cpu().numpy() - ref).max() <= 1e-13 * np.abs(ref).max()
+
+
 def test_band_singular_info_and_single_solve():
     import torch
     from magic_amd import algebra as A

@@ -205,7 +205,7 @@ def test_grid_step_matches_oracle_on_random_fields(l_max):
     (irfft / get_nl / rfft of step_time.py:931-1212) on O(1) random spectral
     fields, through the same Legendre transforms.  l_max=63 gives n_phi/2 = 96
     (radix-3 register pass, compiled plan); l_max=85 gives n_phi/2 = 128
-    (radix-4 register pass, run-time plan only)."""
+    (radix-8 passes)."""
     from oracle.dynamo import OracleRun
     orun = OracleRun(dict(_GRID_CFG, l_max=l_max, n_r_max=9))
     fields = _random_fields((orun.prm.lm_max, 9), 11)
@@ -270,6 +270,28 @@ def test_fused_grid_step_matches_separate_kernels(l_max):
     assert max(e_gen.values()) < 1e-12, e_gen
     assert np.allclose(cf, cref, rtol=1e-12, atol=0), (cf, cref)
     assert np.allclose(cf, cg, rtol=1e-14, atol=0), (cf, cg)
+
+
+@pytest.mark.parametrize("l_max,mh", [(42, 64), (48, 72), (85, 128), (96, 144), (170, 256)])
+def test_grid_step_plan_lengths_match_run_time_plan(l_max, mh):
+    """Row lengths whose compiled plans have radix-8 passes, padded rows or (FP64,
+    n_phi/2 <= 128) the three components of a vector in one pass, against the
+    run-time plan of the same length and the separate kernels: FP64 within 1e-12
+    and 1e-11, FP32 within 1e-6 of each vector's largest coefficient (the bounds of
+    the tests above: the arithmetic per value is the same up to the order of sums)."""
+    from magic_amd.params import Params
+    assert Params(dict(l_max=l_max, n_r_max=17)).n_phi == 2 * mh
+    fused, cf = _radial_loop_outputs(l_max, "fused")
+    for other, tol, ctol in (("generic", 1e-12, 1e-14), ("separate", 1e-11, 1e-12)):
+        ref, cref = _radial_loop_outputs(l_max, other)
+        errs = _rel_errs(fused, ref)
+        assert max(errs.values()) < tol, (other, errs)
+        assert np.allclose(cf, cref, rtol=ctol, atol=0), (other, cf, cref)
+    out, cour = _radial_loop_outputs(l_max, "fused", precision="mixed")
+    ref, cref = _radial_loop_outputs(l_max, "generic", precision="mixed")
+    errs = _rel_errs(out, ref)
+    assert max(errs.values()) < 1e-6, errs
+    assert np.allclose(cour, cref, rtol=1e-6, atol=0), (cour, cref)
 
 
 @pytest.mark.parametrize("name", ["bench16", "c1", "bprdt", "fd2mhd", "fdbpr", "fdanel", "anel21",

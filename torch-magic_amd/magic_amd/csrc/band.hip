@@ -178,17 +178,33 @@ extern "C" int mh_band_factor(double* abd, int* pivot, int* info, int n, int kl,
 // elimination keeps b(k .. k+kl) in a register window and emits x(k-1) kl
 // columns behind the input; the back substitution streams the columns
 // downwards with the window x(k-m .. k-1), m = kl+ku+1, emitting x(k-1) m
-// columns above the input.  Outputs collect in a ring of LDS tiles that is
-// stored as soon as a tile is complete; the forward result is the back
-// substitution's input (in `sol`).  `rows` (optional) orders the rows by
-// degree so that the lanes of a wave share their factors (broadcast loads).
+// columns above the input.  Outputs replace consumed inputs in a ring of two
+// tiles, stored when the tile after the next needs their slot; the forward
+// result is the back substitution's input (in `sol`).  `rows` (optional) orders
+// the rows by degree so that the lanes of a wave share their factors.
 // In place (rhs == sol) is allowed: every tile is read before any output
 // lands on it.
+//
+// One wave per SIMD (65 k recurrences at l_max = 255), so what a wave waits for is
+// not hidden by others.  Within a tile it waits for nothing but its recurrence: the
+// next tile, its row scaling and its factors and pivots (of up to eight degrees, all
+// that 32 ordered rows hold) are requested before the tile is worked on, with
+// unconditional clamped loads, after the stores of the tile before (a wait for the
+// loads would otherwise cover the stores); and the pivots' reciprocals are formed
+// when the factors are staged, so that a step of the back substitution waits for a
+// product and its correction, which give the correctly rounded quotient, instead
+// of a division.  28 KB of LDS at most and below 256 registers: five waves fit on a
+// CU, and 1028 waves are resident at once (with 35 KB or more registers four would
+// have waited for the rest: 390 us).  l_max = 255, n = 512, kl = ku = 3: 407 us ->
+// 280 us (1.1 GB in four passes: 3.9 TB/s of a copy's 5.5), kl = ku = 2: 356 -> 260;
+// l_max = 383, n = 97: 164 -> 119.
 constexpr int kBT = 16;  // columns per tile
 constexpr int kBR = 32;  // rows per wave
+constexpr int kBD = 8;   // degrees per wave whose factors are staged (the first 32 rows hold 8)
+constexpr int kBS = 4;   // columns whose LDS reads may be issued together (registers)
 
 template <int KL, int KU>
-__global__ __launch_bounds__(64) void k_band_solve(const double* __restrict__ abd_all,
+__global__ __launch_bounds__(64, 2) void k_band_solve(const double* __restrict__ abd_all,
                                                    const int* __restrict__ piv_all,
                                                    const double* __restrict__ fac_row,
                                                    const double* __restrict__ fac_col,
@@ -199,136 +215,191 @@ __global__ __launch_bounds__(64) void k_band_solve(const double* __restrict__ ab
   if (when && *when == 0) return;
   constexpr int M = KL + KU + 1;
   constexpr int NR = 2 * KL + KU + 1;
-  constexpr int TP = kBT + 1;                    // padded LDS row (conflict-free columns)
-  constexpr int NO = (M + kBT - 1) / kBT + 1;    // output ring slots (back substitution)
-  constexpr int CR = 64 / kBT;                   // rows per cooperative access
-  constexpr int CI = kBR / CR;                   // cooperative accesses per lane
-  __shared__ double2 tin[kBR][TP];
-  __shared__ double2 tout[NO > 2 ? NO : 2][kBR][TP];
+  constexpr int TP = kBT + 1;     // padded LDS row (conflict-free columns)
+  constexpr int CR = 64 / kBT;    // rows per cooperative access
+  constexpr int CI = kBR / CR;    // cooperative accesses per lane
+  static_assert(64 % kBT == 0 && kBR % CR == 0, "cooperative tile map");
+  static_assert(M <= kBT && kBD == 2 * CR, "two-tile ring, two staging accesses");
+  __shared__ double2 ring[2][kBR][TP];
+  // a tile's factors of the wave's degrees; row M: the pivots' reciprocals (back
+  // substitution), row KL: the pivots' offsets (forward)
+  __shared__ double facs[kBD][M + 1][kBT];
   const int lane = threadIdx.x;
   const int r0 = blockIdx.x * kBR;
-  // this lane's row and component, and its degree's factors
+  // this lane's row and component, and its degree's factors (lanes past the last row
+  // repeat it; nothing of theirs is stored)
   const int row = lane >> 1, comp = lane & 1;
-  const int ri = r0 + row;
-  const int lm = ri < L ? (rows ? rows[ri] : ri) : 0;
-  const int l = lm2l[lm];
+  auto row_of = [&](int r) { const int q = min(r0 + r, L - 1); return rows ? rows[q] : q; };
+  const int l = lm2l[row_of(row)];
   const double* abd = abd_all + (long)l * NR * n;
   const int* pivot = piv_all + (long)l * n;
-  const double* fcl = fac_col ? fac_col + (long)l * n : nullptr;
-  auto in_at = [&](int c) { return reinterpret_cast<const double*>(&tin[row][c])[comp]; };
-  auto out_at = [&](int slot, int pos, double v) {
-    reinterpret_cast<double*>(&tout[slot][row][pos])[comp] = v;
-  };
   // cooperative map: lane -> sub-row cs (rows cs + CR*it) and column cc of a tile
-  static_assert(64 % kBT == 0 && kBR % CR == 0, "cooperative tile map");
   const int cs = lane / kBT, cc = lane % kBT;
-  long cbase[CI];
-  const double* cfr[CI];
-  bool cok[CI];
+  int clm[CI], cl[CI];  // rows and (where a scaling wants them) their degrees
 #pragma unroll
   for (int it = 0; it < CI; ++it) {
-    const int rr = r0 + cs + CR * it;
-    cok[it] = rr < L;
-    const int lmr = cok[it] ? (rows ? rows[rr] : rr) : 0;
-    cbase[it] = (long)lmr * n;
-    cfr[it] = fac_row ? fac_row + (long)lm2l[lmr] * n : nullptr;
+    clm[it] = row_of(cs + CR * it);
+    cl[it] = fac_row || fac_col ? lm2l[clm[it]] : 0;
   }
-  const int ntile = (n + kBT - 1) / kBT;
-  auto coop_load = [&](const double2* src, int tile, bool scale, double2 (&v)[CI]) {
-    const int col = tile * kBT + cc;
+  // the wave's distinct degrees, up to kBD: this lane's slot among them and the degrees
+  // of the slots whose factors it stages (cs and cs + 4)
+  int sl = 0, nd = 0, lq0 = 0, lq1 = 0;
+  unsigned long long left = ~0ull;
+  while (left && nd < kBD) {
+    const int ld = __builtin_amdgcn_readlane(l, (int)__builtin_ctzll(left));
+    const bool mine = l == ld;
+    sl = mine ? nd : sl;
+    if (cs >= nd) lq0 = ld;  // (slots beyond the last repeat it)
+    if (cs + CR >= nd) lq1 = ld;
+    left &= ~__ballot(mine);
+    ++nd;
+  }
+  const bool fast = left == 0;  // otherwise every lane reads its factors from memory
+
+  // (called where addresses are formed: keeps the compiler from holding the 64-bit
+  // offsets of all rows in registers throughout, which would leave one wave per SIMD)
+  auto fresh = [](int& i) __attribute__((always_inline)) { asm volatile("" : "+v"(i)); };
+
+  // Q factor rows from row `row0` on, at columns base .. base + 15, four degrees an access
+  auto fac_load = [&](int row0, int Q, int base, auto& v, auto& w) __attribute__((always_inline)) {
+    const int c = min(max(base + cc, 0), n - 1);
+    fresh(lq0), fresh(lq1);
+    const double* a0 = abd_all + ((long)lq0 * NR + row0) * n + c;
 #pragma unroll
-    for (int it = 0; it < CI; ++it) {
-      v[it] = make_double2(0.0, 0.0);
-      if (cok[it] && col < n) {
-        v[it] = src[cbase[it] + col];
-        if (scale && cfr[it]) v[it] = cscale(v[it], cfr[it][col]);
-      }
+    for (int q = 0; q < Q; ++q) v[q] = a0[(long)q * n];
+    if (nd > CR) {
+      const double* a1 = abd_all + ((long)lq1 * NR + row0) * n + c;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) w[q] = a1[(long)q * n];
     }
   };
-  auto coop_put = [&](const double2 (&v)[CI]) {
+  auto fac_put = [&](int Q, const auto& v, const auto& w) __attribute__((always_inline)) {
 #pragma unroll
-    for (int it = 0; it < CI; ++it) tin[cs + CR * it][cc] = v[it];
+    for (int q = 0; q < Q; ++q) facs[cs][q][cc] = v[q];
+    if (nd > CR)
+#pragma unroll
+      for (int q = 0; q < Q; ++q) facs[cs + CR][q][cc] = w[q];
   };
-  auto coop_store = [&](int slot, int tile) {
+  double2 pre[CI];  // the next tile
+  double prf[CI];   // and its row scaling
+  auto coop_load = [&](const double2* src, int tile, bool scale) __attribute__((always_inline)) {
+    const int col = min(max(tile, 0) * kBT + cc, n - 1);
+#pragma unroll
+    for (int it = 0; it < CI; ++it) {
+      fresh(clm[it]), fresh(cl[it]);
+      pre[it] = src[(long)clm[it] * n + col];
+    }
+    if (scale)
+#pragma unroll
+      for (int it = 0; it < CI; ++it) prf[it] = fac_row[(long)cl[it] * n + col];
+  };
+  auto coop_put = [&](int slot, bool scale) __attribute__((always_inline)) {
+#pragma unroll
+    for (int it = 0; it < CI; ++it)
+      ring[slot][cs + CR * it][cc] = scale ? cscale(pre[it], prf[it]) : pre[it];
+  };
+  auto coop_store = [&](int tile, const double* fcol) __attribute__((always_inline)) {
     const int col = tile * kBT + cc;
 #pragma unroll
     for (int it = 0; it < CI; ++it)
-      if (cok[it] && col < n) sol[cbase[it] + col] = tout[slot][cs + CR * it][cc];
+      if (r0 + cs + CR * it < L && col < n) {
+        const double2 x = ring[tile & 1][cs + CR * it][cc];
+        fresh(clm[it]), fresh(cl[it]);
+        sol[(long)clm[it] * n + col] = fcol ? cscale(x, fcol[(long)cl[it] * n + col]) : x;
+      }
   };
-  double2 pre[CI];
+  // this lane's element of column c of the tile in a slot
+  auto at = [&](int slot, int c) -> double& {
+    return reinterpret_cast<double*>(&ring[slot][row][c])[comp];
+  };
+  const int ntile = (n + kBT - 1) / kBT;
 
   // ---- forward elimination: x = L^-1 P b (rows scaled by fac_row)
-  if (KL > 0) {
-    double W[KL + 1];
+  if constexpr (KL > 0) {
+    const bool scale = fac_row != nullptr;
+    double W[KL + 1], v[KL], w[KL];
+    int pv = 0, pw = 0;
 #pragma unroll
     for (int j = 0; j <= KL; ++j) W[j] = 0.0;
-    // iteration k (1-based): pivot swap, update of b(k+1 .. k+lmk), emit x(k-1)
-    // (full: an interior iteration, k <= n - KL, so every update applies)
-    auto iter = [&](auto full, int k, int slot, int pos) __attribute__((always_inline)) {
-      constexpr bool FULL = decltype(full)::value;
+    // iteration k (1-based): pivot swap, update of b(k+1 .. k+lmk), x(k-1) = W[0]
+    // (full: an interior iteration, k <= n - KL, so every update applies; staged: the
+    // factors are column c of those in LDS)
+    auto iter = [&](auto full, auto staged, int k, int c) __attribute__((always_inline)) {
+      constexpr bool FULL = decltype(full)::value, ST = decltype(staged)::value;
       const int lmk = FULL ? KL : min(KL, n - k);
-      const int lp = pivot[k - 1] - k;
+      const int lp = (ST ? reinterpret_cast<const int*>(&facs[sl][KL][c])[0] : pivot[k - 1]) - k;
       // swap W[0] and W[lp] with selects (an indexed swap would put W in scratch)
       const double w0 = W[0];
-      double pv = w0;
+      double p = w0;
 #pragma unroll
       for (int j = 1; j <= KL; ++j) {
         const bool s = j == lp;
-        pv = s ? W[j] : pv;
+        p = s ? W[j] : p;
         W[j] = s ? w0 : W[j];
       }
-      W[0] = pv;
 #pragma unroll
       for (int j = 1; j <= KL; ++j)
-        if (FULL || j <= lmk) W[j] += pv * abd[(long)(M + j - 1) * n + (k - 1)];
-      out_at(slot, pos, W[0]);
+        if (FULL || j <= lmk)
+          W[j] += p * (ST ? facs[sl][j - 1][c] : abd[(long)(M + j - 1) * n + (k - 1)]);
+      at(((k - 1) / kBT) & 1, (k - 1) % kBT) = p;
 #pragma unroll
       for (int j = 0; j < KL; ++j) W[j] = W[j + 1];
       W[KL] = 0.0;
     };
-    int flushed = 0;  // output tiles < flushed are stored
-    auto ftile = [&](int t) __attribute__((always_inline)) {
-      __syncthreads();  // the previous tile's readers are done
-      coop_put(pre);
+    auto fetch = [&](int t) __attribute__((always_inline)) {
+      coop_load(rhs, t, scale);
+      if (fast) {
+        fac_load(M, KL, t * kBT - KL, v, w);
+        const int c = min(max(t * kBT - KL + cc, 0), n - 1);
+        pv = piv_all[(long)lq0 * n + c];
+        if (nd > CR) pw = piv_all[(long)lq1 * n + c];
+      }
+    };
+    fetch(0);
+    for (int t = 0; t < ntile; ++t) {
+      const int slot = t & 1;
+      __syncthreads();  // the previous tile's outputs are in the ring
+      if (t >= 2) coop_store(t - 2, nullptr);
       __syncthreads();
-      if (t + 1 < ntile) coop_load(rhs, t + 1, true, pre);
+      coop_put(slot, scale);
+      if (fast) {
+        fac_put(KL, v, w);
+        reinterpret_cast<int*>(&facs[cs][KL][cc])[0] = pv;
+        if (nd > CR) reinterpret_cast<int*>(&facs[cs + CR][KL][cc])[0] = pw;
+      }
+      __syncthreads();
+      fetch(min(t + 1, ntile - 1));
       if (t >= 1 && (t + 1) * kBT <= n) {
-        // interior tile: straight-line iterations (their loads can be issued early)
+        // interior tile: straight-line iterations (iteration k emits column k - 1,
+        // KL behind the column that enters)
+        auto tile = [&](auto staged) __attribute__((always_inline)) {
 #pragma unroll
-        for (int c = 0; c < kBT; ++c) {
-          W[KL] = in_at(c);
-          const int o = t * kBT + c - KL;
-          iter(std::true_type{}, o + 1, (o / kBT) & 1, (c - KL + kBT) % kBT);
-        }
+          for (int c = 0; c < kBT; ++c) {
+            W[KL] = at(slot, c);
+            iter(std::true_type{}, staged, t * kBT + c - KL + 1, c);
+            if (c % kBS == kBS - 1) __builtin_amdgcn_sched_barrier(0);
+          }
+        };
+        if (fast) tile(std::true_type{});
+        else tile(std::false_type{});
       } else {
-#pragma unroll
-      for (int c = 0; c < kBT; ++c) {
-        const int j = t * kBT + c;  // input column entering the window
-        if (j < n) {
-          W[KL] = in_at(c);
-          if (j >= KL) {
-            // iteration k = j - KL + 1 emits column j - KL
-            const int o = j - KL;
-            iter(std::false_type{}, o + 1, (o / kBT) & 1, (c - KL + kBT) % kBT);
-          } else {
+#pragma unroll 1
+        for (int c = 0; c < kBT; ++c) {
+          const int j = t * kBT + c;  // input column entering the window
+          if (j >= n) break;
+          W[KL] = at(slot, c);
+          if (j < KL) {
             // filling: b(0 .. KL-1) move down as they arrive
 #pragma unroll
             for (int q = 0; q < KL; ++q) W[q] = W[q + 1];
+          } else if (fast) {
+            iter(std::false_type{}, std::true_type{}, j - KL + 1, c);
+          } else {
+            iter(std::false_type{}, std::false_type{}, j - KL + 1, 0);
           }
         }
       }
-      }
-      // outputs so far cover columns <= hi: store every complete tile (a tile's
-      // ring slot is written again only two input tiles later)
-      const int hi = min(t * kBT + kBT - 1, n - 1) - KL;
-      __syncthreads();
-      while (flushed < ntile && flushed * kBT + kBT - 1 <= hi) {
-        coop_store(flushed & 1, flushed);
-        ++flushed;
-      }
-    };
-    coop_load(rhs, 0, true, pre);
-    for (int t = 0; t < ntile; ++t) ftile(t);
+    }
     // fewer columns than KL: finish the fill with zeros
     for (int j = n; j < KL; ++j) {
 #pragma unroll
@@ -336,90 +407,114 @@ __global__ __launch_bounds__(64) void k_band_solve(const double* __restrict__ ab
       W[KL] = 0.0;
     }
     // the last iterations (nothing left to enter), then x(n-1) = W[0]
-    for (int k = max(1, n - KL + 1); k <= n - 1; ++k) {
-      const int o = k - 1;
-      iter(std::false_type{}, k, (o / kBT) & 1, o % kBT);
-    }
-    out_at(((n - 1) / kBT) & 1, (n - 1) % kBT, W[0]);
+    for (int k = max(1, n - KL + 1); k <= n - 1; ++k)
+      iter(std::false_type{}, std::false_type{}, k, 0);
+    at(((n - 1) / kBT) & 1, (n - 1) % kBT) = W[0];
     __syncthreads();
-    while (flushed < ntile) {
-      coop_store(flushed & 1, flushed);
-      ++flushed;
-    }
+    if (ntile > 1) coop_store(ntile - 2, nullptr);
+    coop_store(ntile - 1, nullptr);
   }
 
   // ---- back substitution: x = U^-1 y (columns scaled by fac_col)
   {
     const double2* src = (KL > 0) ? sol : rhs;
-    const bool scale_in = (KL == 0);  // without a forward pass the row scaling is applied here
-    double V[M];
+    const bool scale = KL == 0 && fac_row;  // without a forward pass the row scaling is applied here
+    double V[M], v[M], w[M];
 #pragma unroll
     for (int j = 0; j < M; ++j) V[j] = 0.0;
     // iteration k (1-based, descending): finish x(k-1), update x(k-2 .. k-1-lmk)
     // (full: k > M, so every update applies)
-    auto biter = [&](auto full, int k) __attribute__((always_inline)) {
-      constexpr bool FULL = decltype(full)::value;
-      V[M - 1] /= abd[(long)(M - 1) * n + (k - 1)];
+    auto iter = [&](auto full, auto staged, int k, int c) __attribute__((always_inline)) {
+      constexpr bool FULL = decltype(full)::value, ST = decltype(staged)::value;
+      double x;
+      if (ST) {
+        const double d = facs[sl][M - 1][c], r = facs[sl][M][c], q = V[M - 1] * r;
+        x = fma(fma(-q, d, V[M - 1]), r, q);
+        x = fabs(q) < INFINITY ? x : q;
+      } else {
+        x = V[M - 1] / abd[(long)(M - 1) * n + (k - 1)];
+      }
       const int lmk = FULL ? M - 1 : min(k, M) - 1;
-      const double t = -V[M - 1];
 #pragma unroll
       for (int j = 1; j < M; ++j)
-        if (FULL || j <= lmk) V[M - 1 - j] += t * abd[(long)(M - j - 1) * n + (k - 1)];
-      const int o = k - 1;
-      out_at((o / kBT) % NO, o % kBT, fcl ? V[M - 1] * fcl[o] : V[M - 1]);
+        if (FULL || j <= lmk)
+          V[M - 1 - j] += -x * (ST ? facs[sl][M - j - 1][c] : abd[(long)(M - j - 1) * n + (k - 1)]);
+      at(((k - 1) / kBT) & 1, (k - 1) % kBT) = x;
 #pragma unroll
       for (int j = M - 1; j > 0; --j) V[j] = V[j - 1];
       V[0] = 0.0;
     };
-    int flushed = ntile;  // output tiles >= flushed are stored
-    auto btile = [&](int u) __attribute__((always_inline)) {
+    auto fetch = [&](int u) __attribute__((always_inline)) {
+      coop_load(src, u, scale);
+      if (fast) fac_load(0, M, u * kBT + M, v, w);  // (u = -1: the last M steps)
+    };
+    // stages the factors and the pivots' reciprocals; false when a pivot is so small or
+    // so large that a product with its reciprocal is not to be trusted
+    auto stage = [&]() __attribute__((always_inline)) {
+      auto usable = [](double d) { return fabs(d) > 0x1p-900 && fabs(d) < 0x1p900; };
+      fac_put(M, v, w);
+      bool ok = usable(v[M - 1]);
+      facs[cs][M][cc] = 1.0 / v[M - 1];
+      if (nd > CR) {
+        ok = ok && usable(w[M - 1]);
+        facs[cs + CR][M][cc] = 1.0 / w[M - 1];
+      }
+      return (bool)__all(ok);
+    };
+    bool st = false;
+    fetch(ntile - 1);
+    for (int u = ntile - 1; u >= 0; --u) {
+      const int slot = u & 1;
+      __syncthreads();  // the previous tile's outputs are in the ring
+      if (u + 2 < ntile) coop_store(u + 2, fac_col);
       __syncthreads();
-      coop_put(pre);
+      coop_put(slot, scale);
+      if (fast) st = stage();
       __syncthreads();
-      if (u > 0) coop_load(src, u - 1, scale_in, pre);
+      fetch(u - 1);
       if ((u + 1) * kBT + M <= n) {
-        // interior tile: straight-line iterations (k = col + M + 1 <= n, k > M)
+        // interior tile: straight-line iterations (k = column + M + 1 <= n, k > M)
+        auto tile = [&](auto staged) __attribute__((always_inline)) {
 #pragma unroll
-        for (int c = kBT - 1; c >= 0; --c) {
-          const double v = in_at(c);
-          biter(std::true_type{}, u * kBT + c + M + 1);
-          V[0] = v;
-        }
+          for (int c = kBT - 1; c >= 0; --c) {
+            const double y = at(slot, c);
+            iter(std::true_type{}, staged, u * kBT + c + M + 1, c);
+            V[0] = y;
+            if (c % kBS == 0) __builtin_amdgcn_sched_barrier(0);
+          }
+        };
+        if (st) tile(std::true_type{});
+        else tile(std::false_type{});
       } else {
-#pragma unroll
-      for (int c = kBT - 1; c >= 0; --c) {
-        const int col = u * kBT + c;  // input column entering the window from below
-        if (col < n) {
-          const double v = in_at(c);
+#pragma unroll 1
+        for (int c = kBT - 1; c >= 0; --c) {
+          const int col = u * kBT + c;  // input column entering the window from below
+          if (col >= n) continue;
+          const double y = at(slot, c);
           const int k = col + M + 1;
           if (k <= n) {
-            biter(std::false_type{}, k);
-            V[0] = v;
+            if (st) iter(std::false_type{}, std::true_type{}, k, c);
+            else iter(std::false_type{}, std::false_type{}, k, 0);
+            V[0] = y;
           } else {
             // initial fill of x(n-1) .. x(n-M), by distance from the top
             const int pos = M - 1 - (n - 1 - col);
 #pragma unroll
             for (int j = 0; j < M; ++j)
-              if (j == pos) V[j] = v;
+              if (j == pos) V[j] = y;
           }
         }
       }
-      }
-      // outputs so far cover columns >= u*kBT + M: store every complete tile
-      __syncthreads();
-      while (flushed - 1 >= 0 && (flushed - 1) * kBT >= u * kBT + M) {
-        --flushed;
-        coop_store(flushed % NO, flushed);
-      }
-    };
-    coop_load(src, ntile - 1, scale_in, pre);
-    for (int u = ntile - 1; u >= 0; --u) btile(u);
-    for (int k = min(M, n); k >= 1; --k) biter(std::false_type{}, k);
-    __syncthreads();
-    while (flushed - 1 >= 0) {
-      --flushed;
-      coop_store(flushed % NO, flushed);
     }
+    __syncthreads();
+    if (fast) st = stage();
+    __syncthreads();
+    for (int k = min(M, n); k >= 1; --k)
+      if (st) iter(std::false_type{}, std::true_type{}, k, kBT - 1 - M + k);
+      else iter(std::false_type{}, std::false_type{}, k, 0);
+    __syncthreads();
+    if (ntile > 1) coop_store(1, fac_col);
+    coop_store(0, fac_col);
   }
 }
 
