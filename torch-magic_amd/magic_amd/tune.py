@@ -1,16 +1,16 @@
 """Launch-shape tuner.
 
-Two launch shapes are chosen by timing on the device, once per shape and
+The launch shapes below are chosen by timing on the device, once per shape and
 precision, because the best one depends on the sizes and every choice gives
 the same results bit for bit:
 
 * the fused grid step (``mh_grid_step``): radial levels per workgroup, 1, 2,
   ... up to the most its FFT plan fits (``mh_grid_plan``);
-* the Legendre synthesis (``mh_leg_synth``): waves per workgroup, 4 or 6
+* the FP32 and BF16 Legendre synthesis (``mh_leg_synth``): waves per workgroup, 4 or 6
   (16 theta pairs each), and for the FP32 vector synthesis one or two column
   tiles per workgroup; the vector and the scalar synthesis are tuned apart;
-* the Legendre analysis (``mh_leg_analysis``): waves per workgroup, 6 or 4
-  (16 degrees each);
+* the FP32 Legendre analysis (``mh_leg_analysis``): waves per workgroup, 6 or 4
+  (16 degrees each; FP64 has a work split of its own, a rule on the sizes);
 * the row operator (``mh_rowop``): tiles of 32 rows x 64 or x 128 columns.
 
 Choices are remembered in memory for the process and in a JSON file
@@ -193,7 +193,10 @@ def rowop_wide(run) -> int:
 
 
 def grid_key(res, N: int, fprec: int, l_mag: bool) -> str:
-    return f"{_device_name(res)}|grid_step|Mh={res.Mh}|T={res.T}|M={res.M}|N={N}|fprec={fprec}|mag={int(l_mag)}"
+    # a choice holds for the kernels it was timed with: files written before the radix-8
+    # and batched FP64 plans hold 4 levels where 1 is the best now (l_max = 85, 49 levels:
+    # 231 against 109 us), so the key names the kernels' generation
+    return f"{_device_name(res)}|grid_step/2|Mh={res.Mh}|T={res.T}|M={res.M}|N={N}|fprec={fprec}|mag={int(l_mag)}"
 
 
 def grid_level_block(res, N: int, p, fdtype=torch.float64, bufs=None, reps: int = 3) -> int:
