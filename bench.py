@@ -56,16 +56,15 @@ NOISE = dict(seed=20261202, amp=1e-4)
 # keyed by the tuner's radial levels per workgroup (0: the plan's own block, four
 # levels for the FP32 grid step at n_phi = 1152; the FP64 step chose one); other
 # level blocks have no measured figure (traffic null).  The FP32 Legendre entries
-# ("mixed") are from the same kernels profiled before the BF16 headline.
+# ("mixed") are from the same kernels profiled before the BF16 headline; the FP64
+# Legendre kernels have no figure.
 PMC_TRAFFIC_BYTES = {
     ("grid_step", "mixed", 0): 2.540e9 + 1.791e9,
     ("grid_step", "fp64", 1): 5.861e9 + 4.554e9,
     ("leg_syn_vec", "mixed_bf16x3"): 3.444e9 + 2.171e9,
     ("leg_syn_vec", "mixed"): 4.196e9 + 2.192e9,
-    ("leg_syn_vec", "fp64"): 5.721e9 + 4.187e9,
     ("leg_ana_vec", "mixed_bf16x3"): 1.640e9 + 0.601e9,
     ("leg_ana_vec", "mixed"): 1.414e9 + 0.599e9,
-    ("leg_ana_vec", "fp64"): 7.779e9 + 0.620e9,
 }
 
 PEAK_FP64_TFLOPS = 78.6
@@ -95,11 +94,12 @@ def section_work(p, N, fbytes=16.0):
     Nb = N - 2
     return {
         # Legendre: 4 flops per real-matrix x complex-coefficient multiply-add
-        # with the equatorial fold (one H-length product per (l, m))
-        "leg_syn_vec": ("mfma", 20.0 * L * H * 4 * N),
+        # with the equatorial fold (one H-length product per (l, m)); FP64 vector transforms
+        # take three products a (Q, S, T) group and two a pair, FP32 and BF16 five and four
+        "leg_syn_vec": ("mfma", (12.0 if fbytes == 16.0 else 20.0) * L * H * 4 * N),
         "leg_syn_scal": ("mfma", 4.0 * L * H * N),
         "leg_ana_scal": ("mfma", 4.0 * L * H * 3 * Nb),
-        "leg_ana_vec": ("mfma", 16.0 * L * H * 3 * Nb),
+        "leg_ana_vec": ("mfma", (8.0 if fbytes == 16.0 else 16.0) * L * H * 3 * Nb),
         # per-degree fused solves: (3N x N) on 4 systems, (6N x 2N) on (w, p)
         "rowop_szbj": ("mfma", 4 * 12.0 * L * N * N),
         "rowop_wp": ("mfma", 48.0 * L * N * N),
@@ -622,8 +622,8 @@ def main():
                               else "fp64_gemm_TFLOPs"]}[rl["unit"]]
         if rl["unit"] == "TFLOP/s" and head in ("mixed_bf16", "mixed_bf16x3") and \
                 rl["kernel"].startswith("leg_"):
-            meas = float("nan")   # no BF16 GEMM is measured
-        rl["frac_of_measured_peak"] = rl["achieved"] / meas
+            meas = None   # no BF16 GEMM is measured
+        rl["frac_of_measured_peak"] = rl["achieved"] / meas if meas else None
         print("bench: measured peaks done", file=sys.stderr, flush=True)
     cpu = None
     if not args.no_cpu_baseline:
