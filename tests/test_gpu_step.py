@@ -170,13 +170,16 @@ def _random_fields(shape, seed):
     return {k: rng.standard_normal(shape) + 1j * rng.standard_normal(shape) for k in _FIELDS}
 
 
-def _radial_loop_outputs(l_max, mode, seed=11, precision="fp64"):
-    """One radial loop on random spectral fields; mode: fused, generic or separate."""
+def _radial_loop_outputs(l_max, mode, seed=11, precision="fp64", rb=None):
+    """One radial loop on random spectral fields; mode: fused, generic or separate;
+    rb: radial levels per workgroup of the grid step (the tuner's by default)."""
     import torch
     from magic_amd.dynamo import DynamoRun
     run = DynamoRun(dict(_GRID_CFG, l_max=l_max, n_r_max=9, precision=precision),
                     fused_grid=(mode != "separate"))
     run.grid_generic = mode == "generic"
+    if rb is not None:
+        run.grid_rb = rb
     for k, a in _random_fields(tuple(run.f["s"].shape), seed).items():
         run.f[k].copy_(torch.as_tensor(a))
     cour = run.radial_loop()
@@ -272,23 +275,25 @@ def test_fused_grid_step_matches_separate_kernels(l_max):
     assert np.allclose(cf, cg, rtol=1e-14, atol=0), (cf, cg)
 
 
+@pytest.mark.parametrize("rb", [0, 1, 2])
 @pytest.mark.parametrize("l_max,mh", [(42, 64), (48, 72), (85, 128), (96, 144), (170, 256)])
-def test_grid_step_plan_lengths_match_run_time_plan(l_max, mh):
+def test_grid_step_plan_lengths_match_run_time_plan(l_max, mh, rb):
     """Row lengths whose compiled plans have radix-8 passes, padded rows or (FP64,
-    n_phi/2 <= 128) the three components of a vector in one pass, against the
-    run-time plan of the same length and the separate kernels: FP64 within 1e-12
-    and 1e-11, FP32 within 1e-6 of each vector's largest coefficient (the bounds of
-    the tests above: the arithmetic per value is the same up to the order of sums)."""
+    n_phi/2 <= 128, one or two levels) the three components of a vector in one pass,
+    against the run-time plan of the same length and the separate kernels, at the
+    level blocks that have a kernel of their own: FP64 within 1e-12 and 1e-11, FP32
+    within 1e-6 of each vector's largest coefficient (the bounds of the tests above:
+    the arithmetic per value is the same up to the order of sums)."""
     from magic_amd.params import Params
     assert Params(dict(l_max=l_max, n_r_max=17)).n_phi == 2 * mh
-    fused, cf = _radial_loop_outputs(l_max, "fused")
+    fused, cf = _radial_loop_outputs(l_max, "fused", rb=rb)
     for other, tol, ctol in (("generic", 1e-12, 1e-14), ("separate", 1e-11, 1e-12)):
-        ref, cref = _radial_loop_outputs(l_max, other)
+        ref, cref = _radial_loop_outputs(l_max, other, rb=0)
         errs = _rel_errs(fused, ref)
         assert max(errs.values()) < tol, (other, errs)
         assert np.allclose(cf, cref, rtol=ctol, atol=0), (other, cf, cref)
-    out, cour = _radial_loop_outputs(l_max, "fused", precision="mixed")
-    ref, cref = _radial_loop_outputs(l_max, "generic", precision="mixed")
+    out, cour = _radial_loop_outputs(l_max, "fused", precision="mixed", rb=rb)
+    ref, cref = _radial_loop_outputs(l_max, "generic", precision="mixed", rb=0)
     errs = _rel_errs(out, ref)
     assert max(errs.values()) < 1e-6, errs
     assert np.allclose(cour, cref, rtol=1e-6, atol=0), (cour, cref)
@@ -523,13 +528,13 @@ def test_device_step_control_replays_schedule_with_timers():
     assert "step_ctl" in t and "rebuild" in t
 
 
-@pytest.mark.parametrize("l_max,precision", [(32, "fp64"), (32, "mixed"), (63, "fp64"),
-                                             (85, "mixed"), (383, "mixed"), (383, "fp64")])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("l_max", [20, 32, 40, 42, 48, 63, 72, 85, 96, 127, 170, 191, 255, 383])
 def test_grid_level_blocks_give_identical_results(l_max, precision):
-    """Every level block the tuner may choose (1, 2, 4, ... up to the plan's own)
-    gives the same Fourier outputs and Courant maxima bit for bit: compiled plans
-    (n_phi 96, 192, 1152, with their 1- and 2-level instantiations) and the
-    run-time plan (n_phi 256, and the other counts)."""
+    """Every level block the tuner may choose (1, 2, 4, ... up to the plan's own), and
+    blocks between those, give the same Fourier outputs and Courant maxima bit for
+    bit: compiled plans (n_phi/2 = 48, 64, 72, 96, 128, 144, 192, 256, 288, 384, 576,
+    their own, 1- and 2-level instantiations) and the run-time plan (30, 60, 108)."""
     import torch
     from magic_amd import tune
     from magic_amd.device import Resolution
@@ -546,7 +551,7 @@ def test_grid_level_blocks_give_identical_results(l_max, precision):
                      dtype=fdt) * 1e-2
     own = res.grid_plan()[2]
     outs = {}
-    for rb in tune.grid_candidates(own):
+    for rb in sorted({*tune.grid_candidates(own), min(3, own), max(1, own - 1)}):
         Fo = res.fourier_buffer(9, N - 2, fdt).zero_()
         cfl = torch.zeros(2 * N, dtype=torch.int64, device="cuda")
         res.grid_step(Fs, Fv, Fo, N, cfl, p, rb=0 if rb == own else rb)

@@ -18,9 +18,9 @@ constexpr int kLdsBytes = 160 * 1024 - 256;
 // levels per workgroup.  LDS: two buffers of RB rows of LS complex values,
 // then the twiddles exp(-2 pi i k/Mh) and exp(-2 pi i k/(2Mh)), k < Mh.
 //
-// Two kinds of LDS passes (wide_plan() chooses): radix 4, or (`wide`) radix 8 with
-// odd radices first, one pass, one barrier and a fifth of the LDS traffic less
-// (Mh = 576: 3, 8, 8 and the register radix 3, against 4, 4, 4, 3).  Wide passes, and
+// Two kinds of LDS passes in compiled plans (wide_plan() chooses): radix 4, or (`wide`)
+// radix 8 with odd radices first, one pass, one barrier and a fifth of the LDS traffic
+// less (Mh = 576: 3, 8, 8 and the register radix 3, against 4, 4, 4, 3).  Wide passes, and
 // the passes behind an odd radix, pad: a pass writes groups of Ns*R elements, and one
 // element of padding after each group keeps lanes that write the same place of
 // consecutive groups on different banks; it costs the next pass nothing, whose Ns is
@@ -30,9 +30,6 @@ struct GPlan {
   int radix[16];
   int LS;  // LDS row length
   bool pad;
-  // ceil(2^32 / d) of the run-time plan's divisors, x / d = umulhi(x, m) for x < 2^16:
-  // butterflies per row of each pass, and its Ns in the inverse and forward order
-  unsigned mnb[16], mni[16], mnf[16];
 };
 
 // Whether a padding plan pads groups of `group` elements: even groups of 8 to 32 (an
@@ -41,7 +38,9 @@ struct GPlan {
 constexpr bool pads(int group) { return group % 2 == 0 && group >= 8 && group <= 32; }
 
 // Half lengths with a compiled plan (all divisions and stage loops resolved
-// at compile time); other lengths run the same code with the run-time plan.
+// at compile time); other lengths run the same code with the run-time plan, which has
+// neither radix 8 nor padding: in the run-time kernel they spill (FP64: 50 to 160
+// registers).
 #define MH_GRID_COMPILED(X) \
   X(24) X(48) X(64) X(72) X(96) X(128) X(144) X(192) X(256) X(288) X(384) X(576) X(768)
 constexpr bool grid_compiled(int Mh) {
@@ -54,6 +53,11 @@ constexpr bool grid_compiled(int Mh) {
   }
 }
 
+// Radix of the register pass (0: no plan).
+constexpr int register_radix(int Mh) {
+  return Mh % 3 == 0 ? 3 : Mh % 4 == 0 ? 4 : Mh % 2 == 0 ? 2 : Mh % 5 == 0 ? 5 : 0;
+}
+
 // Kind of plan, by length and element size only, so that every level block, batched
 // or not, compiled or not, gives the same results bit for bit.  Wide where three
 // components are transformed together in workgroups of some waves: their 9/8
@@ -63,17 +67,20 @@ constexpr bool grid_compiled(int Mh) {
 // single component of one level (long FP64 rows) has 72 butterflies for 192 threads
 // (l_max = 383: 4.34 against 4.72 ms).
 constexpr bool wide_plan(int Mh, int esz) {
-  return grid_compiled(Mh) && Mh >= 128 && (esz == 4 || Mh <= 128);
+  return Mh >= 128 && (esz == 4 || Mh <= 128);
 }
 
-constexpr GPlan make_plan(int Mh, bool wide = false) {
+// The plan of a compiled kernel for elements of `esz` bytes per real, or (esz = 0) the
+// run-time plan.
+constexpr GPlan make_plan(int Mh, int esz = 0) {
   GPlan p{};
   if (Mh < 2) return p;
-  const int RL = Mh % 3 == 0 ? 3 : Mh % 4 == 0 ? 4 : Mh % 2 == 0 ? 2 : Mh % 5 == 0 ? 5 : 0;
+  const int RL = register_radix(Mh);
   if (RL == 0) return p;
+  const bool wide = esz > 0 && wide_plan(Mh, esz);
   int n = Mh / RL, k = 0;
   // odd radices first in padding plans: their first pass writes at an odd stride
-  p.pad = wide || (grid_compiled(Mh) && n % 3 == 0);
+  p.pad = wide || (esz > 0 && n % 3 == 0);
   while (p.pad && n % 3 == 0 && k < 15) { p.radix[k++] = 3; n /= 3; }
   while (wide && n % 8 == 0 && k < 15) { p.radix[k++] = 8; n /= 8; }
   while (n % 4 == 0 && k < 15) { p.radix[k++] = 4; n /= 4; }
@@ -93,14 +100,6 @@ constexpr GPlan make_plan(int Mh, bool wide = false) {
     if (p.pad && pads(dn) && Mh + Mh / dn + 2 > p.LS) p.LS = Mh + Mh / dn + 2;
   }
   p.LS += p.LS % 2;
-  for (int s = 0, up = 1, dn = 1; s < k; ++s) {
-    const int f = k - 1 - s;
-    p.mnb[s] = (unsigned)(((1ull << 32) + Mh / p.radix[s] - 1) / (Mh / p.radix[s]));
-    p.mni[s] = up > 1 ? (unsigned)(((1ull << 32) + up - 1) / up) : 0u;
-    p.mnf[f] = dn > 1 ? (unsigned)(((1ull << 32) + dn - 1) / dn) : 0u;
-    up *= p.radix[s];
-    dn *= p.radix[f];
-  }
   for (int rb = 16; rb >= 1; --rb) {
     const int th = (rb * p.TP + 63) / 64 * 64;
     if (th <= kMaxThreads && (2 * rb * p.LS + 2 * Mh) * 16 <= kLdsBytes) {
@@ -113,6 +112,19 @@ constexpr GPlan make_plan(int Mh, bool wide = false) {
   return p;
 }
 
+#define MH_CREG(V) static_assert(register_radix(V) == 3 || register_radix(V) == 4, "launch_generic");
+MH_GRID_COMPILED(MH_CREG)
+#undef MH_CREG
+
+// Whether a compiled plan transforms three components together: always in FP32; in
+// FP64 for short rows with one or two levels per workgroup, where barriers bound the
+// passes (two levels: l_max = 16, 33 levels 27 -> 20 us; l_max = 64, 65 levels 100 -> 85
+// us), while long rows lose more workgroups per CU to the LDS and registers of three
+// than the barriers cost (l_max = 383, 97 levels: 5.5 ms against 4.3 one by one).
+constexpr bool grid_batched(int Mh, int rbc, int esz) {
+  return esz == 4 || (Mh <= 128 && (rbc == 1 || rbc == 2));
+}
+
 // Workgroup barrier that waits for this wave's LDS operations only, so the
 // global loads of the next component stay in flight across FFT passes.
 __device__ __forceinline__ void lds_barrier() {
@@ -122,7 +134,8 @@ __device__ __forceinline__ void lds_barrier() {
 extern __shared__ double2 g_lds_raw[];
 
 // Geometry of one launch; compile-time constants when MH > 0.  MH = 0 runs a run-time
-// plan without radix 8 and padding, MH = -1 one with them.
+// plan; MH = -1 the plan of a compiled length with its radix 8 and padding (the check
+// of the compiled kernels that MhGridArgs.generic asks for).
 struct Geo {
   int Mh, M, RB, LS, TP, nst, threads;
   bool pad;
@@ -134,7 +147,7 @@ __device__ __forceinline__ Geo make_geo(const GridArgs& a, const GPlan& rp) {
   Geo g;
   g.M = a.M;
   if constexpr (MH > 0) {
-    constexpr GPlan P = make_plan(MH, wide_plan(MH, sizeof(T)));
+    constexpr GPlan P = make_plan(MH, sizeof(T));
     g.Mh = MH;
     g.RB = RBC > 0 ? RBC : P.RB;
     g.TP = P.TP;
@@ -147,7 +160,7 @@ __device__ __forceinline__ Geo make_geo(const GridArgs& a, const GPlan& rp) {
     g.RB = rp.RB;
     g.TP = rp.TP;
     g.nst = rp.nst;
-    g.LS = rp.LS;
+    g.LS = MH < 0 ? rp.LS : g.Mh + 2;
     g.pad = MH < 0 && rp.pad;
     g.threads = rp.threads;
   }
@@ -185,22 +198,21 @@ struct Ctx {
 // by the rule of pads() (a group of one, the packed spectrum, has none).
 template <int R, typename T, bool PAD>
 __device__ __forceinline__ void stage_mid(const Geo& g, const GridArgs& a, int win, int wout, int Ns,
-                                          double dir, int nrows, unsigned mnb = 0, unsigned mns = 0) {
+                                          double dir, int nrows) {
   typedef typename vec2<T>::type V;
   const int nb = g.Mh / R, tstep = g.Mh / (Ns * R);
   const bool pin = PAD && pads(Ns), pout = PAD && pads(Ns * R);
-  const int rstep = pin ? nb + nb / Ns : nb, gstep = Ns * R + (pout ? 1 : 0);
+  const int rstep = pin ? nb + nb / Ns : nb;
   const V* tw = ltw<T>(g);
   const V* in = lbuf<T>(g, win);
   V* out = lbuf<T>(g, wout);
   for (int idx = threadIdx.x; idx < nrows * nb; idx += g.threads) {
-    // run-time divisors by their reciprocals (a division takes some 25 instructions)
-    const int row = mnb ? (int)__umulhi((unsigned)idx, mnb) : idx / nb, bf = idx - row * nb;
-    const int gr = Ns == 1 ? bf : mns ? (int)__umulhi((unsigned)bf, mns) : bf / Ns, k = bf - gr * Ns;
-    const V* src = in + row * g.LS + bf + (pin ? gr : 0);
+    const int row = idx / nb, bf = idx - row * nb;
+    const int k = bf % Ns;
+    const V* src = in + row * g.LS + (pin ? bf / Ns : 0);
     V v[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = src[r * rstep];
+    for (int r = 0; r < R; ++r) v[r] = src[bf + r * rstep];
     if (Ns > 1) {
       // powers of w by products from one table value (exp(-i...); the inverse
       // conjugates), for radix 8 from w and w^2, so that none is more than
@@ -230,8 +242,8 @@ __device__ __forceinline__ void stage_mid(const Geo& g, const GridArgs& a, int w
       }
     }
     dft_any<R>(v, dir);
-    V* dst = out + row * g.LS + gr * gstep + k;
-    if constexpr (sizeof(T) == 4 && R == 4) {
+    V* dst = out + row * g.LS + (bf / Ns) * Ns * R + (pout ? bf / Ns : 0) + k;
+    if constexpr (sizeof(T) == 4 && (R == 2 || R == 4)) {
       if (Ns == 1) {
         // consecutive outputs from an even element: 16-byte stores of pairs
         // (half the store instructions at this pass's stride of R values)
@@ -246,24 +258,22 @@ __device__ __forceinline__ void stage_mid(const Geo& g, const GridArgs& a, int w
   }
 }
 
-// Run-time radix; radix 8 and padding only where WIDE: its registers would spill in
-// the kernels that never use it.
+// Run-time radix; radix 8 and padding only where WIDE.
 template <typename T, bool WIDE>
 __device__ __forceinline__ void stage_mid_rt(const Geo& g, const GridArgs& a, int R, int win, int wout,
-                                             int Ns, double dir, int nrows, unsigned mnb,
-                                             unsigned mns) {
+                                             int Ns, double dir, int nrows) {
   if (WIDE && R == 8) {
-    if constexpr (WIDE) stage_mid<8, T, WIDE>(g, a, win, wout, Ns, dir, nrows, mnb, mns);
-  } else if (R == 4) stage_mid<4, T, WIDE>(g, a, win, wout, Ns, dir, nrows, mnb, mns);
-  else if (R == 2) stage_mid<2, T, WIDE>(g, a, win, wout, Ns, dir, nrows, mnb, mns);
-  else if (R == 3) stage_mid<3, T, WIDE>(g, a, win, wout, Ns, dir, nrows, mnb, mns);
-  else stage_mid<5, T, WIDE>(g, a, win, wout, Ns, dir, nrows, mnb, mns);
+    if constexpr (WIDE) stage_mid<8, T, WIDE>(g, a, win, wout, Ns, dir, nrows);
+  } else if (R == 4) stage_mid<4, T, WIDE>(g, a, win, wout, Ns, dir, nrows);
+  else if (R == 2) stage_mid<2, T, WIDE>(g, a, win, wout, Ns, dir, nrows);
+  else if (R == 3) stage_mid<3, T, WIDE>(g, a, win, wout, Ns, dir, nrows);
+  else stage_mid<5, T, WIDE>(g, a, win, wout, Ns, dir, nrows);
 }
 
 // Inverse stages 0 .. nst-2 of a compiled plan (S = stage, NS = its Ns).
 template <int MH, int S, int NS, typename T>
 __device__ __forceinline__ int inv_mid_ct(const Geo& g, const GridArgs& a, int w, int nrows) {
-  constexpr GPlan P = make_plan(MH, wide_plan(MH, sizeof(T)));
+  constexpr GPlan P = make_plan(MH, sizeof(T));
   if constexpr (S < P.nst - 1) {
     constexpr int R = P.radix[S];
     stage_mid<R, T, P.pad>(g, a, w, 1 - w, NS, 1.0, nrows);
@@ -277,7 +287,7 @@ __device__ __forceinline__ int inv_mid_ct(const Geo& g, const GridArgs& a, int w
 // Forward stages S = nst-2 .. 0 of a compiled plan.
 template <int MH, int S, int NS, typename T>
 __device__ __forceinline__ int fwd_mid_ct(const Geo& g, const GridArgs& a, int w, int nrows) {
-  constexpr GPlan P = make_plan(MH, wide_plan(MH, sizeof(T)));
+  constexpr GPlan P = make_plan(MH, sizeof(T));
   if constexpr (S >= 0) {
     constexpr int R = P.radix[S];
     stage_mid<R, T, P.pad>(g, a, w, 1 - w, NS, -1.0, nrows);
@@ -327,15 +337,6 @@ __device__ __forceinline__ void fetch(const Geo& g, const GridArgs& a, Prefetch<
   }
 }
 
-// Whether a compiled plan transforms three components together: always in FP32; in
-// FP64 for short rows with one or two levels per workgroup, where barriers bound the
-// passes (two levels: l_max = 16, 33 levels 27 -> 20 us; l_max = 64, 65 levels 100 -> 85
-// us), while long rows lose more workgroups per CU to the LDS and registers of three
-// than the barriers cost (l_max = 383, 97 levels: 5.5 ms against 4.3 one by one).
-constexpr bool grid_batched(int Mh, int rbc, int esz) {
-  return esz == 4 || (Mh <= 128 && (rbc == 1 || rbc == 2));
-}
-
 struct NoFetch {
   __device__ void operator()() const {}
 };
@@ -383,8 +384,7 @@ __device__ __forceinline__ void inverse(Ctx& c, const Geo& g, const GridArgs& a,
       const GPlan& P = *c.rp;
       int Ns = 1;
       for (int s = 0; s < P.nst - 1; ++s) {
-        stage_mid_rt<T, MH < 0>(g, a, P.radix[s], w, 1 - w, Ns, 1.0, g.RB,
-                                     P.mnb[s], P.mni[s]);
+        stage_mid_rt<T, MH < 0>(g, a, P.radix[s], w, 1 - w, Ns, 1.0, g.RB);
         Ns *= P.radix[s];
         w = 1 - w;
         lds_barrier();
@@ -432,14 +432,13 @@ __device__ __forceinline__ void forward(Ctx& c, const Geo& g, const GridArgs& a,
   }
   lds_barrier();
   if constexpr (MH > 0) {
-    constexpr GPlan P = make_plan(MH, wide_plan(MH, sizeof(T)));
+    constexpr GPlan P = make_plan(MH, sizeof(T));
     w = fwd_mid_ct<MH, P.nst - 2, RL, T>(g, a, w, g.RB);
   } else {
     const GPlan& P = *c.rp;
     int Ns = RL;
     for (int s = P.nst - 2; s >= 0; --s) {
-      stage_mid_rt<T, MH < 0>(g, a, P.radix[s], w, 1 - w, Ns, -1.0, g.RB,
-                                   P.mnb[s], P.mnf[s]);
+      stage_mid_rt<T, MH < 0>(g, a, P.radix[s], w, 1 - w, Ns, -1.0, g.RB);
       Ns *= P.radix[s];
       w = 1 - w;
       lds_barrier();
@@ -479,8 +478,8 @@ __device__ __forceinline__ void forward(Ctx& c, const Geo& g, const GridArgs& a,
 }
 
 // ---------------------------------------------------------------- batched transforms
-// The FP32 kernel of the compiled plans transforms the three components of a
-// vector (u, B, curl u, curl B; the three outputs of each product) together:
+// k_grid_step3 transforms the three components of a vector (u, B, curl u, curl B;
+// the three outputs of each product) together:
 // component k of level j is LDS row k*RB + j, and every LDS pass runs over the
 // 3*RB rows, so a vector costs the barriers of one transform instead of three.
 // Each row's arithmetic is that of the single-component transform.
@@ -603,7 +602,7 @@ __device__ __forceinline__ void forwardN(Ctx& c, const Geo& g, const GridArgs& a
   }
   lds_barrier();
   {
-    constexpr GPlan P = make_plan(MH, wide_plan(MH, sizeof(T)));
+    constexpr GPlan P = make_plan(MH, sizeof(T));
     w = fwd_mid_ct<MH, P.nst - 2, RL, T>(g, a, w, NC * RB);
   }
   const int Mh = g.Mh, N = a.N, No = N - 2, n = (Mh / 2 + 1) * RB;
@@ -1058,8 +1057,6 @@ __global__ __launch_bounds__((plan_threads<MH, RBC>()), (sizeof(T) == 4 ? 3 : 2)
     atomicMax(a.cfl + h * N + r0 + j, red[h * RB + j]);
   }
 }
-
-// Compiled plan for the common half lengths, run-time plan otherwise.
 
 // Launch of a compiled plan with RBC levels per workgroup (0: the plan's own);
 // false when Mh has no compiled plan.
