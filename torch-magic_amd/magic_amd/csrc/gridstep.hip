@@ -69,7 +69,7 @@ extern "C" int mh_grid_step(const MhGridArgs* args, void* stream) {
   if (a.N < 3 || a.T < 1 || a.Mh < 2 || a.M < 1 || a.M > a.Mh) return MH_EINVAL;
   if (a.fprec != 0 && a.fprec != 1) return MH_EINVAL;
   const int esz = a.fprec ? 4 : 8;
-  bool compiled = !a.generic && grid_compiled(a.Mh);
+  const bool compiled = !a.generic && grid_compiled(a.Mh);
   GPlan P = make_plan(a.Mh, grid_compiled(a.Mh) ? esz : 0);
   if (P.RL == 0) return MH_EINVAL;
   // level block: the plan's own (the most levels that fit), or a.rb fewer; the compiled
@@ -88,12 +88,8 @@ extern "C" int mh_grid_step(const MhGridArgs* args, void* stream) {
   // component (M orders) below 2^31 elements
   if ((long)a.T * 4 * a.N * 2 >= (1L << 24) || (long)a.M * a.T * 4 * a.N * 2 >= (1L << 31))
     return MH_EINVAL;
-  const auto lds_of = [&](int comps) {
-    return (2ull * comps * P.RB * P.LS + 2ull * a.Mh) * 2 * esz;
-  };
-  bool batched = compiled && grid_batched(a.Mh, rb == own_rb ? 0 : rb, esz);
-  if (batched && lds_of(3) > (size_t)kLdsBytes) compiled = batched = false;
-  const size_t lds = lds_of(batched ? 3 : 1);
+  const bool batched = compiled && grid_batched(a.Mh, rb == own_rb ? 0 : rb, esz);
+  const size_t lds = (2ull * (batched ? 3 : 1) * P.RB * P.LS + 2ull * a.Mh) * 2 * esz;
   if (lds > (size_t)kLdsBytes) return MH_EINVAL;
   const int nRB = (a.N + P.RB - 1) / P.RB;
   const long nwg = (long)a.T * nRB;

@@ -112,17 +112,39 @@ constexpr GPlan make_plan(int Mh, int esz = 0) {
   return p;
 }
 
+// Callers ask for level blocks by the run-time plan (mh_grid_plan): every plan of a
+// length has the same block, threads and register pass.
+constexpr bool same_block(int Mh, int esz) {
+  const GPlan p = make_plan(Mh), c = make_plan(Mh, esz);
+  return p.RB == c.RB && p.threads == c.threads && p.RL == c.RL && p.TP == c.TP;
+}
+#define MH_CSAME(V) static_assert(same_block(V, 4) && same_block(V, 8), "level block of the plans");
+MH_GRID_COMPILED(MH_CSAME)
+#undef MH_CSAME
 #define MH_CREG(V) static_assert(register_radix(V) == 3 || register_radix(V) == 4, "launch_generic");
 MH_GRID_COMPILED(MH_CREG)
 #undef MH_CREG
 
-// Whether a compiled plan transforms three components together: always in FP32; in
-// FP64 for short rows with one or two levels per workgroup, where barriers bound the
-// passes (two levels: l_max = 16, 33 levels 27 -> 20 us; l_max = 64, 65 levels 100 -> 85
-// us), while long rows lose more workgroups per CU to the LDS and registers of three
-// than the barriers cost (l_max = 383, 97 levels: 5.5 ms against 4.3 one by one).
+// Threads and LDS bytes of a compiled kernel with RBC levels per workgroup (0: the
+// plan's own) and `comps` components transformed together.
+constexpr int plan_threads(int Mh, int rbc, int esz) {
+  const GPlan p = make_plan(Mh, esz);
+  return rbc > 0 ? (rbc * p.TP + 63) / 64 * 64 : p.threads;
+}
+constexpr long plan_lds(int Mh, int rbc, int esz, int comps) {
+  const GPlan p = make_plan(Mh, esz);
+  return (2L * comps * (rbc > 0 ? rbc : p.RB) * p.LS + 2L * Mh) * 2 * esz;
+}
+
+// Whether a compiled plan transforms three components together: in FP32 where they
+// fit the LDS (all but the own block of 12 levels at 256); in FP64 for short rows
+// with one or two levels per workgroup, where barriers bound the passes (two levels:
+// l_max = 16, 33 levels 27 -> 20 us; l_max = 64, 65 levels 100 -> 85 us), while long rows
+// lose more workgroups per CU to the LDS and registers of three than the barriers
+// cost (l_max = 383, 97 levels: 5.5 ms against 4.3 one by one).
 constexpr bool grid_batched(int Mh, int rbc, int esz) {
-  return esz == 4 || (Mh <= 128 && (rbc == 1 || rbc == 2));
+  return (esz == 4 || (Mh <= 128 && (rbc == 1 || rbc == 2))) &&
+         plan_lds(Mh, rbc, esz, 3) <= kLdsBytes;
 }
 
 // Workgroup barrier that waits for this wave's LDS operations only, so the
@@ -857,16 +879,12 @@ __global__ __launch_bounds__(kMaxThreads, 3) void k_grid_step(GridArgs a, GPlan 
   }
 }
 
-// FP32 grid step of the compiled plans with the vector components transformed
-// together (inverseN / forwardN over 3*RB LDS rows).  Same arithmetic per
-// value as k_grid_step<MH, RL, float, RBC>, in the same order.
-template <int MH, int RBC>
-constexpr int plan_threads() {
-  return RBC > 0 ? (RBC * make_plan(MH).TP + 63) / 64 * 64 : make_plan(MH).threads;
-}
-
+// Grid step of the compiled plans with the vector components transformed together
+// (inverseN / forwardN over 3*RB LDS rows), where grid_batched().  Same arithmetic per
+// value as k_grid_step<MH, RL, T, RBC>, in the same order.
 template <int MH, int RL, typename T, int RBC>
-__global__ __launch_bounds__((plan_threads<MH, RBC>()), (sizeof(T) == 4 ? 3 : 2)) void k_grid_step3(
+__global__ __launch_bounds__(plan_threads(MH, RBC, sizeof(T)),
+                             (sizeof(T) == 4 ? 3 : 2)) void k_grid_step3(
     GridArgs a, GPlan rp) {
   typedef typename vec2<T>::type V;
   __shared__ unsigned long long red[2 * 16];
