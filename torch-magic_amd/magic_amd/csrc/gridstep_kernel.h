@@ -58,16 +58,24 @@ constexpr int register_radix(int Mh) {
   return Mh % 3 == 0 ? 3 : Mh % 4 == 0 ? 4 : Mh % 2 == 0 ? 2 : Mh % 5 == 0 ? 5 : 0;
 }
 
-// Kind of plan, by length and element size only, so that every level block, batched
-// or not, compiled or not, gives the same results bit for bit.  Wide where three
-// components are transformed together in workgroups of some waves: their 9/8
-// butterflies per thread cost a second round to one wave in eight (FP32, l_max = 383,
-// 97 levels: 2.77 -> 2.38 ms; l_max = 85, FP64: 114 -> 108 us); in one or two waves the
-// second round is the whole pass again (l_max = 64, FP32: 50 against 55 us), and a
-// single component of one level (long FP64 rows) has 72 butterflies for 192 threads
-// (l_max = 383: 4.34 against 4.72 ms).
+// Whether a compiled plan has wide passes: by length and element size only, so that
+// every level block gives the same results bit for bit.  Times below: us at 33 / 97
+// levels with the best level block, radix 4 -> radix 8.
+// FP32 from 128 on, where the plan's own block gains as well as the best one (128: 47 ->
+// 45 / 98 -> 94; 192: 82 -> 82 / 225 -> 218; 256: 132 -> 130 / 382 -> 377; 288: 206 -> 191 / 563 ->
+// 525; 384: 361 -> 343 / 1012 -> 953; 576: 934 -> 816 / 2673 -> 2354; 768: 1645 -> 1478 / 5103 ->
+// 4571; 144 loses, 60 -> 61 / 119 -> 121).  Below it the sides differ by block: 96 gains
+// with two levels (40 -> 36) and loses with its own eight (45 -> 51), 72 gains 12 %, 24, 48
+// and 64 0 to 6 %.
+// FP64: the rows of three components whose register pass has radix 4.  One level's
+// radix-8 butterflies (3 Mh / 8: 24 and 48 of its wave's 64 lanes) are one round, radix 4
+// takes one and a half (64: 33 -> 32 / 58 -> 55; 128: 82 -> 79 / 193 -> 187).  With register
+// radix 3 two levels are the better block and take a second round (96: 47 -> 56 / 112 ->
+// 109); single components (longer rows) have too few butterflies for their threads and
+// more registers (192: 158 -> 161 / 396 -> 401; 256: 260 -> 316 / 710 -> 871; 576: 1483 -> 1596 /
+// 4125 -> 4406; 288, 384 and 768 would gain 4 to 6 %).
 constexpr bool wide_plan(int Mh, int esz) {
-  return Mh >= 128 && (esz == 4 || Mh <= 128);
+  return esz == 4 ? Mh >= 128 : Mh <= 128 && register_radix(Mh) == 4;
 }
 
 // The plan of a compiled kernel for elements of `esz` bytes per real, or (esz = 0) the
