@@ -84,6 +84,28 @@ constexpr WPlan make_wplan(int Mh) {
 #define MH_WFFT_COMPILED(X) \
   X(24) X(48) X(64) X(96) X(128) X(192) X(256) X(288) X(384) X(512) X(576) X(768)
 
+constexpr bool wave_compiled(int Mh) {
+  switch (Mh) {
+#define MH_WC(V) case V:
+    MH_WFFT_COMPILED(MH_WC)
+#undef MH_WC
+    return true;
+    default: return false;
+  }
+}
+
+// Whether rows of length Mh, `nstage` radix-2 to 5 passes, are transformed by single
+// waves: compiled plans, run-time plans from 100 on, and below that those with half the
+// passes (72: 9 x 8 for 4 x 2 x 3 x 3).  Short rows are a few elements a lane, and the
+// run-time passes' index arithmetic costs more than the workgroup's barriers that they
+// save (k_fft_inverse -> k_wfft_inverse, 8 columns: 30 5.7 -> 7.5 us, 60 7.3 -> 7.5, 80 8.3 ->
+// 9.0, 90 10.0 -> 10.4; 72 9.1 -> 7.0, 100 9.9 -> 8.0, 120 12.0 -> 7.8).
+constexpr bool wave_rows(int Mh, int nstage) {
+  if (wave_compiled(Mh)) return true;
+  const int nst = make_wplan(Mh).nst;
+  return nst > 0 && (Mh >= 100 || 2 * nst <= nstage);
+}
+
 // Geometry and plan of a launch: compile-time constants when MH > 0.
 template <int MH>
 struct WGeo {
@@ -212,7 +234,7 @@ __device__ __forceinline__ void wave_passes_ct(int li, const double2* __restrict
 
 }  // namespace
 
-// F -> G as k_fft_inverse below, for Mh <= 768.
+// F -> G as k_fft_inverse below.
 template <int MH>
 __global__ __launch_bounds__(512, MH > 0 ? 4 : 2) void k_wfft_inverse(FftArgs a, WPlan pa) {
   extern __shared__ double2 lds[];
@@ -256,16 +278,12 @@ __global__ __launch_bounds__(512, MH > 0 ? 4 : 2) void k_wfft_inverse(FftArgs a,
   }
   __syncthreads();
   const int j = threadIdx.x >> p.lsh, li = threadIdx.x & (p.lpr - 1);
-  if (j >= RB) return;
+  if (j >= nrow) return;  // rows past the batch
   double2* row = lds + j * p.S;
-  const bool act = j < nrow;
-  double2* G = reinterpret_cast<double2*>(a.G + c * a.Gc_stride +
-                                          ((long)(bs + (act ? j : 0)) * a.T + t) * 2L * Mh);
+  double2* G = reinterpret_cast<double2*>(a.G + c * a.Gc_stride + ((long)(bs + j) * a.T + t) * 2L * Mh);
   auto ld = [&](int e) { return row[e + (e >> p.psh)]; };
   auto st = [&](int e, double2 v) { row[e + (e >> p.psh)] = v; };
-  auto out = [&](int e, double2 v) {
-    if (act) G[e] = v;
-  };
+  auto out = [&](int e, double2 v) { G[e] = v; };
   if constexpr (MH > 0) {
     wave_passes_ct<MH, 0, 1>(li, tw, 1.0, ld, ld, st, out);
   } else {
@@ -278,7 +296,7 @@ __global__ __launch_bounds__(512, MH > 0 ? 4 : 2) void k_wfft_inverse(FftArgs a,
   }
 }
 
-// G -> F as k_fft_forward below, for Mh <= 768.
+// G -> F as k_fft_forward below.
 template <int MH>
 __global__ __launch_bounds__(512, MH > 0 ? 4 : 2) void k_wfft_forward(FftArgs a, WPlan pa) {
   extern __shared__ double2 lds[];
@@ -291,11 +309,12 @@ __global__ __launch_bounds__(512, MH > 0 ? 4 : 2) void k_wfft_forward(FftArgs a,
   const double2* tw2 = TW2(a);
   {
     const int j = threadIdx.x >> p.lsh, li = threadIdx.x & (p.lpr - 1);
-    if (j < RB) {
+    // (the compiled plans work on the first row again instead of branching around the
+    // passes: l_max = 383, 97 columns 198 against 207 us)
+    if (j < (MH > 0 ? RB : nrow)) {
       double2* row = lds + j * p.S;
-      const bool act = j < nrow;
       const double2* G = reinterpret_cast<const double2*>(
-          a.G + c * a.Gc_stride + ((long)(bs + (act ? j : 0)) * a.T + t) * 2L * Mh);
+          a.G + c * a.Gc_stride + ((long)(bs + (j < nrow ? j : 0)) * a.T + t) * 2L * Mh);
       auto in = [&](int e) { return G[e]; };
       auto ld = [&](int e) { return row[e + (e >> p.psh)]; };
       auto st = [&](int e, double2 v) { row[e + (e >> p.psh)] = v; };
@@ -342,8 +361,9 @@ static void wfft_launch(int forward, const FftArgs& a, const WPlan& p, hipStream
   else hipLaunchKernelGGL((k_wfft_inverse<MH>), grid, blk, bytes, st, a, p);
 }
 
-// ---------------------------------------------------------------- long rows
-// Workgroup-wide transforms for the rows that do not fit a wave's registers.
+// ---------------------------------------------------------------- workgroup rows
+// Workgroup-wide transforms for the rows that do not fit a wave's registers and for
+// short rows without a compiled plan (wave_rows()).
 
 // F (spectral) -> G (grid): x_j = sum_k X_k e^{+2 pi i jk/n}, X_{n-k} = conj(X_k).
 __global__ __launch_bounds__(256) void k_fft_inverse(FftArgs a) {
@@ -432,10 +452,17 @@ extern "C" int mh_fft(int forward, const MhFftArgs* args, void* stream) {
     prod *= R;
   }
   if (prod != a.Mh) return MH_EINVAL;
-  WPlan p = make_wplan(a.Mh);
-  while (p.rsh > 0 && (p.RB >> 1) >= a.B) p.RB = 1 << --p.rsh;  // no rows past a short batch
-  if (p.nst > 0) {
+  const size_t lds = 2ull * a.RB * a.Mh * sizeof(double2);
+  if (lds > 160 * 1024) return MH_EINVAL;
+  if (wave_rows(a.Mh, a.nstage)) {
     if ((long)a.B * a.T * a.ncomp >= 0x7fffffffL) return MH_EINVAL;
+    WPlan p = make_wplan(a.Mh);
+    while (p.rsh > 0 && (p.RB >> 1) >= a.B) p.RB = 1 << --p.rsh;  // no rows past a short batch
+    // the run-time passes take 159 registers, so that a workgroup of eight whole waves is
+    // alone on its CU: four rows there (Mh = 400: 9 columns 41 -> 25 us, 97 229 -> 175 inverse
+    // and 204 -> 152 forward; compiled plans lose up to 9 % of the forward transform to
+    // the shorter runs of F)
+    if (!wave_compiled(a.Mh) && p.lsh == 6 && p.rsh > 2) p.RB = 1 << (p.rsh = 2);
     switch (a.Mh) {
 #define MH_WCASE(V) case V: wfft_launch<V>(forward, a, p, mh_stream(stream)); break;
       MH_WFFT_COMPILED(MH_WCASE)
@@ -444,8 +471,6 @@ extern "C" int mh_fft(int forward, const MhFftArgs* args, void* stream) {
     }
     return mh_launch_status();
   }
-  const size_t lds = 2ull * a.RB * a.Mh * sizeof(double2);
-  if (lds > 160 * 1024) return MH_EINVAL;
   dim3 grid(mh_cdiv(a.B, a.RB), a.T, a.ncomp);
   if (forward)
     hipLaunchKernelGGL(k_fft_forward, grid, dim3(256), lds, mh_stream(stream), a);
