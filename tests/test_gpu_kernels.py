@@ -354,6 +354,44 @@ def test_fp64_transforms_at_tile_edges(l_max, B, minc):
         assert np.abs(a.cpu().numpy() - b).max() < tol * np.abs(b).max()
 
 
+@pytest.mark.parametrize("l_max,B", [(16, 1500), (27, 20), (31, 300), (48, 520), (85, 300), (91, 210),
+                                     (127, 200), (200, 41), (341, 40)])
+def test_fp64_work_splits_give_identical_results(l_max, B):
+    """The FP64 Legendre kernels choose their work split by sizes and batch: one or
+    three column tiles of the scalar synthesis (three from B > 16 where the launch is
+    large, as at these B), one to three theta tiles a wave (l_max 16, 48, 127), and the
+    analysis of few columns or low degrees (two windows from l_max = 31, four from 91).
+    Every column of a large batch equals the column in a small one bit for bit."""
+    torch = _torch()
+    from magic_amd.params import Params
+    from magic_amd.device import Resolution
+    from magic_amd.sht import SHT
+    res = Resolution(Params({"l_max": l_max, "n_r_max": 9}))
+    sht = SHT(res)
+    gen = torch.Generator(device="cuda").manual_seed(l_max)
+    x = [torch.randn(res.L, B, dtype=torch.complex128, device="cuda", generator=gen) for _ in range(3)]
+    g = [torch.randn(B, res.T, res.P, dtype=torch.float64, device="cuda", generator=gen)
+         for _ in range(2)]
+    big = (sht.scal_to_spat(x[0]), *sht.torpol_to_spat(*x))
+    ana = (sht.scal_to_SH(g[0]), *sht.spat_to_sphertor(*g))
+    for c in (slice(0, 1), slice(3, 11), slice(B - 9, B), slice(0, 16), slice(B - 17, B)):
+        y = [v[:, c].contiguous() for v in x]
+        part = (sht.scal_to_spat(y[0]), *sht.torpol_to_spat(*y))
+        assert all(torch.equal(a[c], b) for a, b in zip(big, part)), c
+        h = [v[c].contiguous() for v in g]
+        part = (sht.scal_to_SH(h[0]), *sht.spat_to_sphertor(*h))
+        assert all(torch.equal(a[:, c], b) for a, b in zip(ana, part)), c
+    # outputs inside wider rows: the columns around them stay as they were
+    F = res.fourier_buffer(4, 7).normal_()
+    for N in (9, 16):
+        out = [torch.full((res.L, N), 5.0, dtype=torch.complex128, device="cuda") for _ in range(3)]
+        p = [o.data_ptr() + 16 for o in out]
+        res.analysis(F, 7, 7, [(0, 1)], p[:1], p[1:2], N, vector=True)
+        res.analysis(F, 7, 7, [2], p[2:], [None], N, vector=False)
+        for o in out:
+            assert (o[:, 0] == 5.0).all() and (o[:, 8:] == 5.0).all() and (o[:, 1:8] != 5.0).all()
+
+
 @pytest.mark.parametrize("Mh", [2, 3, 5, 12, 24, 30, 45, 48, 64, 72, 81, 90, 96, 100, 128, 150, 192,
                                 225, 288, 300, 384, 400, 500, 576, 648, 720, 768, 800, 1000])
 def test_fft_lengths_match_numpy(Mh):

@@ -239,10 +239,11 @@ int leg_synth_f64(int vector, const SynArgs& a, int n_m, hipStream_t st) {
   // with six, 2.86 with four, 3.01 with two; l_max = 127, 6 tiles: 136, 159, 147 us)
   const int nt = mh_cdiv(a.H, 16), ny0 = mh_cdiv(nt, 6), NT = mh_cdiv(mh_cdiv(nt, ny0), 2);
   const int ny = mh_cdiv(nt, 2 * NT);
-  // scalar fields: three column tiles per workgroup once that leaves enough
-  // workgroups for the 256 CUs, one tile otherwise
+  // scalar fields: three column tiles per workgroup where the batch has them and that
+  // leaves enough workgroups for the 256 CUs, one tile otherwise (l_max = 341: 8 columns
+  // in three tiles 42 us, in one 27; 17 columns 46 and 50)
   const long rows = (long)n_m * ny * a.ngroups;
-  const bool three = vector || rows * mh_cdiv(a.B, 24) >= 1024;
+  const bool three = vector || (a.B > 16 && rows * mh_cdiv(a.B, 24) >= 1024);
   const long units =
       (long)a.ngroups * mh_cdiv(a.B, !vector && three ? 24 : 8) * ny * mh_cdiv(n_m, 8) * 8;
   if (units > 0x7fffffffL) return MH_EINVAL;
