@@ -24,6 +24,7 @@
 // lane offset that stays fixed or grows by one addition a chunk, and rows
 // before the first degree, past the last one or past the batch are read through
 // buffer descriptors that return zero there, without compares or selects.
+#include <algorithm>
 #include <type_traits>
 
 #include "legendre_common.h"
@@ -38,7 +39,31 @@ __device__ __forceinline__ double2 bld2(__amdgpu_buffer_rsrc_t r, unsigned off) 
   return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
 }
 constexpr unsigned kOut = 0x80000000u;  // an offset past every descriptor
-constexpr int kAnaWindow = 60;          // degree indices per analysis workgroup
+constexpr int kAnaWindow = 60;          // degree indices per entry of the analysis work list
+
+// The neighbour combination of the vector analysis for element v of parity p: `opp`
+// the other parity's sums of this lane, `same` the other field's of this parity, cl =
+// ((l + 1) c_l, l c_{l+1}).  S = l c_{l+1} A_{l+1} - (l + 1) c_l A_{l-1} - i m B_l, and T the first
+// two negated (sgn).
+__device__ __forceinline__ double ana_combine(const double4_t& opp, double same, int p, int v, double sgn,
+                                              double2 cl, double dm, int lane) {
+  // A_{l-1} and A_{l+1}: the other parity at k - 1, k (p = 0) or k, k + 1 (p = 1); a
+  // neighbouring k is the next lane group's element, or the next element of the
+  // group at the other end
+  const int g = lane >> 4;  // accumulator row of element v: g + 4 v
+  const double here = opp[v];
+  double am, ap;
+  if (p == 0) {
+    const double give = g == 3 ? (v > 0 ? opp[v > 0 ? v - 1 : 0] : 0.0) : here;
+    am = __shfl(give, (lane + 48) & 63);
+    ap = here;
+  } else {
+    const double give = g == 0 ? (v < 3 ? opp[v < 3 ? v + 1 : 3] : 0.0) : here;
+    ap = __shfl(give, (lane + 16) & 63);
+    am = here;
+  }
+  return fma(sgn * cl.y, ap, fma(-sgn * cl.x, am, imul_pair(same, -dm, lane)));
+}
 
 }  // namespace
 
@@ -410,28 +435,11 @@ __global__ __launch_bounds__(256, 4) void k_ana64(AnaArgs a, int n_m) {
           if (st && b < a.B) a.outS[comp][(lms + row) * 2L * a.ldo + 2 * b + (col & 1)] = acc[f][p][v];
         }
       } else {
-        // A_{l-1} and A_{l+1}: the other parity at k - 1, k (p = 0) or k, k + 1
-        // (p = 1); a neighbouring k is the next lane group's element, or the next
-        // element of the group at the other end
-        double am[2], ap[2];
-#pragma unroll
-        for (int f = 0; f < 2; ++f) {
-          const double here = acc[f][1 - p][v];
-          if (p == 0) {
-            const double give = g == 3 ? (v > 0 ? acc[f][1][v > 0 ? v - 1 : 0] : 0.0) : here;
-            am[f] = __shfl(give, (lane + 48) & 63);
-            ap[f] = here;
-          } else {
-            const double give = g == 0 ? (v < 3 ? acc[f][0][v < 3 ? v + 1 : 3] : 0.0) : here;
-            ap[f] = __shfl(give, (lane + 16) & 63);
-            am[f] = here;
-          }
-        }
         const double2 cl = lcf[2 * min(row, n) + 1];  // (l + 1) c_l, l c_{l+1}
         const double l = (double)(mo + row);
         const double inv = l > 0.0 ? 1.0 / (l * (l + 1.0)) : 0.0;
-        const double Sv = cl.y * ap[0] - cl.x * am[0] + imul_pair(acc[1][p][v], -dm, lane);
-        const double Tv = cl.x * am[1] - cl.y * ap[1] + imul_pair(acc[0][p][v], -dm, lane);
+        const double Sv = ana_combine(acc[0][1 - p], acc[1][p][v], p, v, 1.0, cl, dm, lane);
+        const double Tv = ana_combine(acc[1][1 - p], acc[0][p][v], p, v, -1.0, cl, dm, lane);
         const int b = bc0 + (col >> 1);
         if (st && b < a.B) {
           const long off = (lms + row) * 2L * a.ldo + 2 * b + (col & 1);
@@ -443,9 +451,153 @@ __global__ __launch_bounds__(256, 4) void k_ana64(AnaArgs a, int n_m) {
   }
 }
 
+// The same sums for few columns and low degrees, where a launch is as long as one
+// wave's chain of MFMAs: one MFMA a step and wave instead of four.  A workgroup takes 8
+// complex columns; a wave one parity, and one field of a window of 15 indices (VEC:
+// the sums meet in LDS for the combination), or one of two such windows (scalar).  Every
+// sum has the terms and the order of k_ana64's, so both give the same bits.
+template <bool VEC>
+__global__ __launch_bounds__(256, 4) void k_ana64s(AnaArgs a, int n_m, int sub) {
+  constexpr int NF = VEC ? 2 : 1, WIN = VEC ? 15 : 30;  // fields; degree indices per workgroup
+  __shared__ double fs[2][NF][2][kChunk][16];            // [buffer][field][fold: +, -][pair][column]
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nbt = (a.B + 7) / 8, gx = a.ncomp * nbt, tpx = a.ntiles / 8;
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, gs = gx * sub;
+  const int* tl = a.tiles + 3 * (xcd * tpx + slot / gs);
+  const int m = tl[0];
+  if (m >= n_m) return;  // uniform per workgroup
+  const int mo = m * (a.minc > 1 ? a.minc : 1);
+  const int n = a.l_max + 1 - mo;
+  // windows inside each column block, as in k_ana64
+  const int nw = (tl[1] >> 16) * sub, q = tl[1] & 0xffff;
+  const int lin = q * gs + slot % gs, cx = lin / nw;
+  const int k0 = (lin - cx * nw) * WIN;
+  if (k0 > 0 && 2 * k0 + 1 >= n) return;  // uniform per workgroup: no degree <= l_max
+  const int p = w & 1, f = VEC ? w >> 1 : 0;
+  const int kb = VEC ? k0 : k0 + 15 * (w >> 1);
+  const bool active = kb == 0 || 2 * kb + 1 < n;
+  const int comp = cx / nbt, bc0 = (cx - comp * nbt) * 8;
+  const int col = lane & 15, kk = lane >> 4;
+  const int r = threadIdx.x >> 3, cc = threadIdx.x & 7;
+  const unsigned ldb = 16u * (unsigned)a.Bin, bytes = 2u * (unsigned)a.H * ldb;
+  const double* Fm = a.F + m * a.m_stride;
+  const __amdgpu_buffer_rsrc_t rf[2] = {
+      brsrc(Fm + (VEC ? a.cf2[comp] : a.cf1[comp]) * a.c_stride, bytes),
+      brsrc(Fm + a.cf1[comp] * a.c_stride, bytes)};
+  unsigned of = bc0 + cc < a.B ? 2u * r * ldb + 16u * (unsigned)(bc0 + cc) : kOut;
+  double2 rn[NF], rs[NF];
+  auto fetch = [&]() {
+#pragma unroll
+    for (int i = 0; i < NF; ++i) {
+      rn[i] = bld2(rf[i], of);
+      rs[i] = bld2(rf[i], of + ldb);
+    }
+    if (of < kOut) of += 2u * kChunk * ldb;
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < NF; ++i) {
+      *reinterpret_cast<double2*>(&fs[buf][i][0][r][2 * cc]) = cadd(rn[i], rs[i]);
+      *reinterpret_cast<double2*>(&fs[buf][i][1][r][2 * cc]) = csub(rn[i], rs[i]);
+    }
+  };
+  constexpr int D = 8, SPC = kChunk / 4;
+  const int K16 = a.mp_info[m * 8 + 4 * p + 3];
+  const double* tp = a.anaW + a.mp_info[m * 8 + 4 * p + 2];
+  const unsigned to = (unsigned)(kk * K16 + min(kb + col, K16 - 1));
+  const int nsteps = (a.H + 3) / 4;
+  double4_t acc = (double4_t){0, 0, 0, 0};
+  double ring[D];
+  auto tload = [&](int s) { return (tp + 4L * s * K16)[to]; };
+  fetch();
+#pragma unroll
+  for (int d = 0; d < D; ++d) ring[d] = tload(min(d, nsteps - 1));
+  store(0);
+  __syncthreads();
+  const int nch = (a.H + kChunk - 1) / kChunk;
+  auto compute = [&](int ch, auto full) {
+    const double(*const x)[16] = fs[ch & 1][f][p] + kk;
+    double xb[2];
+    xb[0] = x[0][col];
+#pragma unroll
+    for (int s = 0; s < SPC; ++s) {
+      const int t = ch * SPC + s;
+      if (!full && t >= nsteps) break;
+      if (s + 1 < SPC) xb[(s + 1) & 1] = x[4 * (s + 1)][col];
+      acc = mfma_f64(ring[s % D], xb[s & 1], acc);
+      if (full) ring[s % D] = tload(min(t + D, nsteps - 1));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  for (int ch = 0; ch + 1 < nch; ++ch) {
+    fetch();
+    if (active) compute(ch, std::true_type{});  // uniform per wave
+    store((ch & 1) ^ 1);                        // last read before the previous barrier
+    __syncthreads();
+  }
+  if (active) compute(nch - 1, std::false_type{});
+  const int g = lane >> 4;
+  const long lms = a.lm_start[m];
+  const int b = bc0 + (col >> 1);
+  if constexpr (!VEC) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int kl = g + 4 * v, row = 2 * (kb + kl) + p;
+      const bool st = active && row < n && (p ? kl < 15 : (kl > 0 || kb == 0));
+      if (st && b < a.B) a.outS[comp][(lms + row) * 2L * a.ldo + 2 * b + (col & 1)] = acc[v];
+    }
+  } else {
+    // (every wave is active)  The buffer that the last chunk did not use: last read
+    // before the previous barrier
+    double(*const ex)[4][64] = reinterpret_cast<double(*)[4][64]>(&fs[nch & 1][0][0][0][0]);
+    static_assert(sizeof(fs) / 2 >= 16 * 64 * sizeof(double), "exchange of the sums");
+#pragma unroll
+    for (int v = 0; v < 4; ++v) ex[w][v][lane] = acc[v];
+    __syncthreads();
+    double* out = f == 0 ? a.outS[comp] : a.outT[comp];
+    double4_t opp, same;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      opp[v] = ex[2 * f + 1 - p][v][lane];
+      same[v] = ex[2 * (1 - f) + p][v][lane];
+    }
+    const double2* lcf = reinterpret_cast<const double2*>(a.lcf) + 2 * (lms + m);
+    const double sgn = f == 0 ? 1.0 : -1.0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int kl = g + 4 * v, row = 2 * (kb + kl) + p;
+      const bool st = row < n && (p ? kl < 15 : (kl > 0 || kb == 0));
+      const double l = (double)(mo + row);
+      const double inv = l > 0.0 ? 1.0 / (l * (l + 1.0)) : 0.0;
+      const double x = ana_combine(opp, same[v], p, v, sgn, lcf[2 * min(row, n) + 1], (double)mo, lane);
+      if (st && b < a.B && out) out[(lms + row) * 2L * a.ldo + 2 * b + (col & 1)] = x * inv;
+    }
+  }
+}
+
 int leg_analysis_f64(int vector, const AnaArgs& a, hipStream_t st) {
   if (a.lcf == nullptr || a.l_max < 0) return MH_EINVAL;
   if ((long)(a.H + kChunk) * 2 * a.Bin * 16 >= (long)kOut) return MH_EINVAL;
+  // workgroups of k_ana64s per list entry: windows of 15 or 30 of its 60 indices (the
+  // ones at k > 0 have degrees where 2 k + 1 <= l_max)
+  const int win = vector ? 15 : 30, sub = std::min(kAnaWindow / win, 1 + std::max(0, a.l_max - 1) / (2 * win));
+  // k_ana64s where its one MFMA a step and wave ends sooner: one window an order (three
+  // quarters or half of k_ana64's waves have no degree there), few workgroups, and scalar
+  // batches whose last tile of 16 columns is less than half full, as long as that is much
+  // of the batch and the orders are short.  k_ana64 -> k_ana64s, us: scalar l_max = 16, 33
+  // columns 4.4 -> 3.5; 60, 97: 8.3 -> 6.4; at the line 96, 64 (388 workgroups): 10.5 -> 10.3, 97
+  // (679): 14.0 -> 14.8; part tiles 333, 8: 34 -> 29; 192, 33: 26 -> 24 and 216, 33: 31 -> 33; 267, 24:
+  // 36 -> 32 and 383, 24: 80 -> 89.  Vector 16, 33: 5.7 -> 4.6; 60, 64 (488): 10.5 -> 8.8; three
+  // pairs of 62 (1464): 18.6 -> 20.9; 96, 8 (97): 9.3 -> 7.4, 17 (291): 11.6 -> 11.9.
+  const long wgs = (long)a.ncomp * mh_cdiv(a.B, vector ? 8 : 16) * a.ntiles;
+  const bool small = sub == 1 || (vector ? wgs < (sub < 4 ? 512 : 192)
+                                         : wgs < 400 || ((a.B - 1) % 16 < 8 && a.B * (long)a.l_max <= 6400));
+  if (small) {
+    const dim3 grid((unsigned)(a.ncomp * mh_cdiv(a.B, 8) * a.ntiles * sub)), blk(256);
+    if (vector) hipLaunchKernelGGL((k_ana64s<true>), grid, blk, 0, st, a, a.n_m, sub);
+    else hipLaunchKernelGGL((k_ana64s<false>), grid, blk, 0, st, a, a.n_m, sub);
+    return mh_launch_status();
+  }
   const dim3 grid((unsigned)(a.ncomp * mh_cdiv(a.B, vector ? 8 : 16) * a.ntiles)), blk(256);
   if (vector) hipLaunchKernelGGL((k_ana64<true>), grid, blk, 0, st, a, a.n_m);
   else hipLaunchKernelGGL((k_ana64<false>), grid, blk, 0, st, a, a.n_m);
