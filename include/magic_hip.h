@@ -74,7 +74,8 @@ typedef struct {
                         (l - 1) c_l, (l + 2) c_{l+1}, (l + 1) c_l, l c_{l+1} with c_l = sqrt((l^2 -
                         m^2) / (4 l^2 - 1)), row lm_start[m] + m + (l - m) (m: mode index in the
                         first two) */
-  int l_max, pad1;   /* prec 0 (the x1, x2 and F rows must lie on 16 bytes) */
+  int l_max, pad1;   /* prec 0, which needs lcf and l_max, reads synP alone and takes x1 and
+                        x2 on 16 bytes; any ldx (past 2^31 bytes an order with slower loads) */
 } MhSynArgs;
 
 /* Legendre synthesis on FP64 MFMA: scalar (vector=0) replaces the bmm part of
@@ -102,11 +103,11 @@ typedef struct {
   int prec;  /* as MhSynArgs.prec (anaW/anaWd hold floats for 1, the bf16 tables for 2, 3) */
   int fprec; /* as MhSynArgs.fprec: F holds floats for 1 (needs prec >= 1) */
   int waves; /* waves per workgroup: 0 = default (6), 6 or 4 (4 only for prec >= 2); tiles
-                must hold 16 * waves degrees */
+                must hold 16 * waves degrees (prec 0 chooses by itself) */
   int minc;  /* as MhSynArgs.minc */
   const int* mp16; /* prec >= 2: as MhSynArgs.mp16 */
   const double* lcf; /* prec 0: as MhSynArgs.lcf */
-  int l_max;
+  int l_max;         /* prec 0, which reads anaW alone and takes F on 16 bytes; any Bin */
   int pad1;
 } MhAnaArgs;
 
@@ -152,7 +153,9 @@ typedef struct {
 
 /* Azimuthal real FFT, norm="forward".  forward=0 replaces torch.fft.irfft in
  * sht.py:341,484-486; forward=1 replaces torch.fft.rfft (and the 1/sin^2
- * scaling) in sht.py:371,597-603. */
+ * scaling) in sht.py:371,597-603.  F and G lie on 16 bytes, their strides are even.  RB: rows
+ * per workgroup where a row takes the whole workgroup (2 RB Mh complex values, at most
+ * 160 KB whatever the length); rows that a wave transforms (up to Mh = 768) have their own. */
 int mh_fft(int forward, const MhFftArgs* args, void* stream);
 
 /* ------------------------------------------------------------ grid space */

@@ -392,6 +392,46 @@ def test_fp64_work_splits_give_identical_results(l_max, B):
             assert (o[:, 0] == 5.0).all() and (o[:, 8:] == 5.0).all() and (o[:, 1:8] != 5.0).all()
 
 
+def test_fp64_legendre_rows_past_32_bit_offsets():
+    """The last 9 columns of arrays whose orders span more than 2^31 bytes (l_max = 4, 40
+    and 22.5 million columns, 10 GB each) transform as they do alone, bit for bit:
+    scalar, and vector with every input mode."""
+    torch = _torch()
+    from magic_amd.params import Params
+    from magic_amd.device import Resolution
+    res = Resolution(Params({"l_max": 4, "n_r_max": 9}))
+    B = 9
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    ld = 40_000_000
+    wide = torch.empty(res.L, ld, dtype=torch.complex128, device="cuda")
+    x = torch.randn(res.L, B, dtype=torch.complex128, device="cuda", generator=gen)
+    v = wide[:, ld - B:]
+    v.copy_(x)
+    outs = []
+    for y, ldx in ((v, ld), (x, B)):
+        Fs, Fv = res.fourier_buffer(1, B).fill_(7.0), res.fourier_buffer(3, 2 * B).fill_(7.0)
+        res.synth([[(y, None, 0)]], B, ldx, Fs, B, vector=False)
+        res.synth([[(y, None, 1), (y, None, 0), (y, y, 2)], [(y, None, 0)] * 3], B, ldx, Fv, 2 * B,
+                  vector=True)
+        outs.append((Fs, Fv))
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+    del wide, v
+    torch.cuda.empty_cache()
+    n = 22_500_000
+    wide = torch.empty(res.M * res.T, n, 2, dtype=torch.float64, device="cuda")
+    F = torch.randn(res.M * res.T, B, 2, dtype=torch.float64, device="cuda", generator=gen)
+    wide[:, n - B:].copy_(F)
+    outs = []
+    for G, Bin in ((wide[:, n - B:], n), (F, B)):
+        o = [torch.full((res.L, B), 7.0, dtype=torch.complex128, device="cuda") for _ in range(3)]
+        res.analysis(G, Bin, B, [0], o[:1], [None], B, vector=False)
+        res.analysis(G, Bin, B, [(0, 0)], o[1:2], o[2:], B, vector=True)
+        outs.append(o)
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+    del wide, G
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("Mh", [2, 3, 5, 12, 24, 30, 45, 48, 64, 72, 81, 90, 96, 100, 128, 150, 192,
                                 225, 288, 300, 384, 400, 500, 576, 648, 720, 768, 800, 1000])
 def test_fft_lengths_match_numpy(Mh):

@@ -39,6 +39,11 @@ __device__ __forceinline__ double2 bld2(__amdgpu_buffer_rsrc_t r, unsigned off) 
   return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
 }
 constexpr unsigned kOut = 0x80000000u;  // an offset past every descriptor
+// The same for rows that 32-bit offsets do not reach: row i < n of `ld` bytes.
+__device__ __forceinline__ double2 gld2(const double* p, int i, int n, long ld, int b, int B) {
+  if (i < 0 || i >= n || b >= B) return make_double2(0.0, 0.0);
+  return *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(p) + i * ld + 16L * b);
+}
 constexpr int kAnaWindow = 60;          // degree indices per entry of the analysis work list
 
 // The neighbour combination of the vector analysis for element v of parity p: `opp`
@@ -78,8 +83,9 @@ __device__ __forceinline__ double ana_combine(const double4_t& opp, double same,
 // staged in LDS by parity (double-buffered, one barrier a chunk); the next
 // chunk's inputs are requested before the current chunk's MFMAs, and each table
 // operand is refilled for the next chunk right after its use, so that every
-// load has a whole chunk (4 x NT x NF MFMAs) to arrive.
-template <bool VEC, int NF, int NT>
+// load has a whole chunk (4 x NT x NF MFMAs) to arrive.  BIG: rows past the reach of
+// the descriptors' offsets, with addresses and compares per load.
+template <bool VEC, int NF, int NT, bool BIG = false>
 __global__ __launch_bounds__(256, NT == 3 && NF == 3 ? 2 : 3) void k_syn64(SynArgs a, int n_m) {
   constexpr int CH = 32, SPC = CH / 8;  // degrees and MFMA steps (per parity) of a chunk
   constexpr int NS = VEC ? 1 : NF;      // scalar column tiles staged per item
@@ -128,17 +134,27 @@ __global__ __launch_bounds__(256, NT == 3 && NF == 3 ? 2 : 3) void k_syn64(SynAr
   // raw inputs of the next chunk: Q (or the scalar tiles), S and T at l - 1, l,
   // l + 1, the second input of T, and the coupling coefficients
   double2 x0[NS], s3[3], t3[3], u3[3], cf;
+  int ir = r;  // BIG: row of the item
+  auto big = [&](const double* x, int i, int b) {
+    return gld2(x + lms * 2 * a.ldx, i, n, 16L * a.ldx, b, a.B);
+  };
   auto fetch = [&]() {
 #pragma unroll
-    for (int f = 0; f < NS; ++f) x0[f] = bld2(rQ, oc[f]);
+    for (int f = 0; f < NS; ++f) x0[f] = BIG ? big(iQ.x1, ir, bc0 + 8 * f + cc) : bld2(rQ, oc[f]);
     if constexpr (VEC) {
       cf = bld2(rC, ol);
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
-        const unsigned o = oc[0] + (unsigned)(q - 1) * ld;
-        s3[q] = bld2(rS, o);
-        t3[q] = bld2(rT, o);
-        u3[q] = bld2(rU, o);  // zero without a second input
+        if constexpr (BIG) {
+          s3[q] = big(iS.x1, ir + q - 1, bc0 + cc);
+          t3[q] = big(iT.x1, ir + q - 1, bc0 + cc);
+          u3[q] = two ? big(iT.x2, ir + q - 1, bc0 + cc) : make_double2(0.0, 0.0);
+        } else {
+          const unsigned o = oc[0] + (unsigned)(q - 1) * ld;
+          s3[q] = bld2(rS, o);
+          t3[q] = bld2(rT, o);
+          u3[q] = bld2(rU, o);  // zero without a second input
+        }
       }
     }
   };
@@ -175,6 +191,7 @@ __global__ __launch_bounds__(256, NT == 3 && NF == 3 ? 2 : 3) void k_syn64(SynAr
     for (int f = 0; f < NS; ++f)
       if (oc[f] < kOut) oc[f] += (unsigned)CH * ld;
     ol += 32u * CH;
+    ir += CH;
   };
   double4_t acc[NT][NF];
 #pragma unroll
@@ -257,22 +274,27 @@ __global__ __launch_bounds__(256, NT == 3 && NF == 3 ? 2 : 3) void k_syn64(SynAr
 
 int leg_synth_f64(int vector, const SynArgs& a, int n_m, hipStream_t st) {
   if (a.lcf == nullptr || a.l_max < 0) return MH_EINVAL;
-  // an order's rows are addressed with 32-bit byte offsets below kOut
-  if ((long)(a.l_max + 64) * a.ldx * 16 >= (long)kOut) return MH_EINVAL;
+  // an order's rows are addressed with 32-bit byte offsets below kOut, or else one by one
+  const bool big = (long)(a.l_max + 64) * a.ldx * 16 >= (long)kOut;
   // theta tiles of 16 pairs over workgroups of two, four or six: the fewest
   // workgroups, since each stages the inputs anew (l_max = 383, 18 tiles: 2.59 ms
   // with six, 2.86 with four, 3.01 with two; l_max = 127, 6 tiles: 136, 159, 147 us)
-  const int nt = mh_cdiv(a.H, 16), ny0 = mh_cdiv(nt, 6), NT = mh_cdiv(mh_cdiv(nt, ny0), 2);
+  const int nt = mh_cdiv(a.H, 16), ny0 = mh_cdiv(nt, 6), NT = big ? 2 : mh_cdiv(mh_cdiv(nt, ny0), 2);
   const int ny = mh_cdiv(nt, 2 * NT);
   // scalar fields: three column tiles per workgroup where the batch has them and that
   // leaves enough workgroups for the 256 CUs, one tile otherwise (l_max = 341: 8 columns
   // in three tiles 42 us, in one 27; 17 columns 46 and 50)
   const long rows = (long)n_m * ny * a.ngroups;
-  const bool three = vector || (a.B > 16 && rows * mh_cdiv(a.B, 24) >= 1024);
+  const bool three = vector || (!big && a.B > 16 && rows * mh_cdiv(a.B, 24) >= 1024);
   const long units =
       (long)a.ngroups * mh_cdiv(a.B, !vector && three ? 24 : 8) * ny * mh_cdiv(n_m, 8) * 8;
   if (units > 0x7fffffffL) return MH_EINVAL;
   const dim3 grid((unsigned)units), blk(256);
+  if (big) {
+    if (vector) hipLaunchKernelGGL((k_syn64<true, 3, 2, true>), grid, blk, 0, st, a, n_m);
+    else hipLaunchKernelGGL((k_syn64<false, 1, 2, true>), grid, blk, 0, st, a, n_m);
+    return mh_launch_status();
+  }
 #define MH_SYN64(NT)                                                                           \
   case NT:                                                                                     \
     if (vector) hipLaunchKernelGGL((k_syn64<true, 3, NT>), grid, blk, 0, st, a, n_m);          \
@@ -455,8 +477,9 @@ __global__ __launch_bounds__(256, 4) void k_ana64(AnaArgs a, int n_m) {
 // wave's chain of MFMAs: one MFMA a step and wave instead of four.  A workgroup takes 8
 // complex columns; a wave one parity, and one field of a window of 15 indices (VEC:
 // the sums meet in LDS for the combination), or one of two such windows (scalar).  Every
-// sum has the terms and the order of k_ana64's, so both give the same bits.
-template <bool VEC>
+// sum has the terms and the order of k_ana64's, so both give the same bits.  BIG as in
+// k_syn64.
+template <bool VEC, bool BIG = false>
 __global__ __launch_bounds__(256, 4) void k_ana64s(AnaArgs a, int n_m, int sub) {
   constexpr int NF = VEC ? 2 : 1, WIN = VEC ? 15 : 30;  // fields; degree indices per workgroup
   __shared__ double fs[2][NF][2][kChunk][16];            // [buffer][field][fold: +, -][pair][column]
@@ -486,13 +509,21 @@ __global__ __launch_bounds__(256, 4) void k_ana64s(AnaArgs a, int n_m, int sub) 
       brsrc(Fm + a.cf1[comp] * a.c_stride, bytes)};
   unsigned of = bc0 + cc < a.B ? 2u * r * ldb + 16u * (unsigned)(bc0 + cc) : kOut;
   double2 rn[NF], rs[NF];
+  int ir = 2 * r;  // BIG: northern row of the pair
   auto fetch = [&]() {
 #pragma unroll
     for (int i = 0; i < NF; ++i) {
-      rn[i] = bld2(rf[i], of);
-      rs[i] = bld2(rf[i], of + ldb);
+      if constexpr (BIG) {
+        const double* Fc = Fm + (VEC && i == 0 ? a.cf2[comp] : a.cf1[comp]) * a.c_stride;
+        rn[i] = gld2(Fc, ir, 2 * a.H, 16L * a.Bin, bc0 + cc, a.B);
+        rs[i] = gld2(Fc, ir + 1, 2 * a.H, 16L * a.Bin, bc0 + cc, a.B);
+      } else {
+        rn[i] = bld2(rf[i], of);
+        rs[i] = bld2(rf[i], of + ldb);
+      }
     }
     if (of < kOut) of += 2u * kChunk * ldb;
+    ir += 2 * kChunk;
   };
   auto store = [&](int buf) {
 #pragma unroll
@@ -577,7 +608,8 @@ __global__ __launch_bounds__(256, 4) void k_ana64s(AnaArgs a, int n_m, int sub) 
 
 int leg_analysis_f64(int vector, const AnaArgs& a, hipStream_t st) {
   if (a.lcf == nullptr || a.l_max < 0) return MH_EINVAL;
-  if ((long)(a.H + kChunk) * 2 * a.Bin * 16 >= (long)kOut) return MH_EINVAL;
+  // the rows of an order past the reach of 32-bit byte offsets (as in leg_synth_f64)
+  const bool big = (long)(a.H + kChunk) * 2 * a.Bin * 16 >= (long)kOut;
   // workgroups of k_ana64s per list entry: windows of 15 or 30 of its 60 indices (the
   // ones at k > 0 have degrees where 2 k + 1 <= l_max)
   const int win = vector ? 15 : 30, sub = std::min(kAnaWindow / win, 1 + std::max(0, a.l_max - 1) / (2 * win));
@@ -590,11 +622,13 @@ int leg_analysis_f64(int vector, const AnaArgs& a, hipStream_t st) {
   // 36 -> 32 and 383, 24: 80 -> 89.  Vector 16, 33: 5.7 -> 4.6; 60, 64 (488): 10.5 -> 8.8; three
   // pairs of 62 (1464): 18.6 -> 20.9; 96, 8 (97): 9.3 -> 7.4, 17 (291): 11.6 -> 11.9.
   const long wgs = (long)a.ncomp * mh_cdiv(a.B, vector ? 8 : 16) * a.ntiles;
-  const bool small = sub == 1 || (vector ? wgs < (sub < 4 ? 512 : 192)
+  const bool small = big || sub == 1 || (vector ? wgs < (sub < 4 ? 512 : 192)
                                          : wgs < 400 || ((a.B - 1) % 16 < 8 && a.B * (long)a.l_max <= 6400));
   if (small) {
     const dim3 grid((unsigned)(a.ncomp * mh_cdiv(a.B, 8) * a.ntiles * sub)), blk(256);
-    if (vector) hipLaunchKernelGGL((k_ana64s<true>), grid, blk, 0, st, a, a.n_m, sub);
+    if (big && vector) hipLaunchKernelGGL((k_ana64s<true, true>), grid, blk, 0, st, a, a.n_m, sub);
+    else if (big) hipLaunchKernelGGL((k_ana64s<false, true>), grid, blk, 0, st, a, a.n_m, sub);
+    else if (vector) hipLaunchKernelGGL((k_ana64s<true>), grid, blk, 0, st, a, a.n_m, sub);
     else hipLaunchKernelGGL((k_ana64s<false>), grid, blk, 0, st, a, a.n_m, sub);
     return mh_launch_status();
   }
