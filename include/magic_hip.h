@@ -36,7 +36,9 @@ extern "C" {
  * SHT matrices of sht.py:84-289.  mp_info[(m*2+p)*4 + {0..3}] =
  * {K, syn_off, ana_off, K16} for parity p = (l-m)%2, K degrees up to l_max; the P_lm
  * tables hold the degree l_max + 1 too (one row more where its parity is p).
- * synP ends with 48 Hp finite values past the last row that are read and unused. */
+ * synP ends with 48 Hp finite values past the last row that are read and unused.  A null
+ * table is not written (FP64 transforms read synP and anaW alone; all four are the
+ * source of the FP32 and BF16 tables). */
 int mh_plm_tables(int l_max, int n_m, int minc, int H, int Hp, const double* cos_t, const double* sin_t,
                   const double* wgt, const int* mp_info, double* synP, double* synD,
                   double* anaW, double* anaWd, void* stream);

@@ -392,6 +392,20 @@ def test_fp64_work_splits_give_identical_results(l_max, B):
             assert (o[:, 0] == 5.0).all() and (o[:, 8:] == 5.0).all() and (o[:, 1:8] != 5.0).all()
 
 
+def test_fp64_resolution_holds_no_derivative_tables():
+    """FP64 transforms read the P_lm tables alone, so a resolution keeps the other two
+    only as the FP32 and BF16 copies of a mixed run."""
+    from magic_amd.params import Params
+    from magic_amd.device import Resolution
+    res = Resolution(Params({"l_max": 42, "n_r_max": 9}))
+    big = [k for k, v in vars(res).items() if getattr(v, "nbytes", 0) >= res.anaW.nbytes // 2]
+    assert sorted(big) == ["anaW", "synP"], big
+    synD, anaWd = res.derivative_tables()
+    t = res.f32_tables()
+    assert (t["synD"] == synD.float()).all() and (t["anaWd"] == anaWd.float()).all()
+    assert not {"synD", "anaWd"} & set(vars(res))
+
+
 def test_fp64_legendre_rows_past_32_bit_offsets():
     """The last 9 columns of arrays whose orders span more than 2^31 bytes (l_max = 4, 40
     and 22.5 million columns, 10 GB each) transform as they do alone, bit for bit:

@@ -61,11 +61,11 @@ __global__ void k_plm_tables(int l_max, int minc, int H, int Hp, const double* _
     const int* info = mp_info + (mi * 2 + p) * 4;
     const long so = (long)info[1] + (long)k * Hp + j;
     const long ao = (long)info[2] + (long)j * info[3] + k;
-    synP[so] = P;
-    anaW[ao] = w2pi * P;
+    if (synP) synP[so] = P;
+    if (anaW) anaW[ao] = w2pi * P;
     if (l <= l_max) {
-      synD[so] = dP;
-      anaWd[ao] = w2pi * dP;
+      if (synD) synD[so] = dP;
+      if (anaWd) anaWd[ao] = w2pi * dP;
     }
     pm1 = p0;
     p0 = p1;

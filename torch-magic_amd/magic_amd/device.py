@@ -69,15 +69,12 @@ class Resolution:
         for k in ("or1", "or2", "or3", "or4", "r2", "rgrav", "q", "valri2", "valhi2"):
             self.d[k] = up(self.rad[k])
         self.d["ost2_grid"] = up(self.th["ost2_grid"])
-        # Legendre tables
+        # Legendre tables: P_lm and its weighted copy (FP64 transforms read no others)
+        for k in ("cos_n", "sin_n", "w_n"):
+            self.d[k] = up(self.th[k])
         self.synP = torch.zeros(self.lay["syn_size"], dtype=F64, device=dev)
-        self.synD = torch.zeros_like(self.synP)
         self.anaW = torch.zeros(self.lay["ana_size"], dtype=F64, device=dev)
-        self.anaWd = torch.zeros_like(self.anaW)
-        cos_n, sin_n, w_n = up(self.th["cos_n"]), up(self.th["sin_n"]), up(self.th["w_n"])
-        _lib.call("mh_plm_tables", p.l_max, p.n_m, p.minc, self.H, self.Hp, ptr(cos_n), ptr(sin_n),
-                  ptr(w_n), ptr(self.d["mp_info"]), ptr(self.synP), ptr(self.synD),
-                  ptr(self.anaW), ptr(self.anaWd), stream_handle())
+        self._plm_tables(self.synP, None, self.anaW, None)
         # FFT plan: complex length Mh = n_phi/2, twiddles exp(-2 pi i k/Mh), exp(-2 pi i k/n_phi)
         self.Mh = p.n_phi // 2
         self.radix = grid.fft_radices(self.Mh)
@@ -93,6 +90,25 @@ class Resolution:
         # stream: make them complete before any other stream can read them
         torch.cuda.current_stream(dev).synchronize()
 
+    def _plm_tables(self, synP, synD, anaW, anaWd):
+        p, d = self.p, self.d
+        _lib.call("mh_plm_tables", p.l_max, p.n_m, p.minc, self.H, self.Hp, ptr(d["cos_n"]),
+                  ptr(d["sin_n"]), ptr(d["w_n"]), ptr(d["mp_info"]), ptr(synP), ptr(synD), ptr(anaW),
+                  ptr(anaWd), stream_handle())
+
+    def derivative_tables(self):
+        """(synD, anaWd): sin(theta) dP_lm/dtheta and its weighted copy in FP64, the
+        source of the FP32 and BF16 tables.  Made anew on each call and not kept (175
+        MB each at l_max = 383)."""
+        if getattr(_lib.recording(), "plan", False):
+            raise RuntimeError("derivative_tables: not inside a recorded launch plan")
+        synD, anaWd = torch.zeros_like(self.synP), torch.zeros_like(self.anaW)
+        self._plm_tables(None, synD, None, anaWd)
+        return synD, anaWd
+
+    synD = property(lambda self: self.derivative_tables()[0])
+    anaWd = property(lambda self: self.derivative_tables()[1])
+
     def f32_tables(self):
         """FP32 copies of the four Legendre tables, shared by every run of the
         resolution.  Built eagerly (a run or transform in mixed precision asks
@@ -103,8 +119,9 @@ class Resolution:
                 raise RuntimeError("f32_tables: the FP32 tables must be built before "
                                    "a launch plan is recorded")
             t = {}
-            for k, src in (("synP", self.synP), ("synD", self.synD), ("anaW", self.anaW),
-                           ("anaWd", self.anaWd)):
+            synD, anaWd = self.derivative_tables()
+            for k, src in (("synP", self.synP), ("synD", synD), ("anaW", self.anaW),
+                           ("anaWd", anaWd)):
                 dst = torch.empty(src.numel(), dtype=torch.float32, device=self.device)
                 _lib.call("mh_tables_to_f32", ptr(src), ptr(dst), src.numel(), stream_handle())
                 t[k] = dst
@@ -136,8 +153,9 @@ class Resolution:
             t = dict(mp16=torch.as_tensor(mp16.reshape(-1), dtype=I32).to(self.device))
             for k, n in (("synP", so), ("synD", so), ("anaW", ao), ("anaWd", ao)):
                 t[k] = torch.zeros(max(n, 1), dtype=torch.int16, device=self.device)
-            _lib.call("mh_tables_to_bf16", ptr(self.synP), ptr(self.synD), ptr(self.anaW),
-                      ptr(self.anaWd), ptr(self.d["mp_info"]), ptr(t["mp16"]), len(info), self.H,
+            synD, anaWd = self.derivative_tables()
+            _lib.call("mh_tables_to_bf16", ptr(self.synP), ptr(synD), ptr(self.anaW),
+                      ptr(anaWd), ptr(self.d["mp_info"]), ptr(t["mp16"]), len(info), self.H,
                       self.Hp, np_, ptr(t["synP"]), ptr(t["synD"]), ptr(t["anaW"]),
                       ptr(t["anaWd"]), stream_handle())
             torch.cuda.current_stream(self.device).synchronize()  # shared across streams
@@ -152,7 +170,7 @@ class Resolution:
             return t, ptr(t["mp16"])
         if prec == 1:
             return self.f32_tables(), 0
-        return dict(synP=self.synP, synD=self.synD, anaW=self.anaW, anaWd=self.anaWd), 0
+        return dict(synP=self.synP, synD=None, anaW=self.anaW, anaWd=None), 0
 
     # ------------------------------------------------------------ launchers
     def fstrides(self, Bout):
