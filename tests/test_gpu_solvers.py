@@ -117,6 +117,37 @@ def test_band_solve_tiles_and_degrees_per_wave(kl, ku, n, scale):
                 assert np.abs(out.cpu().numpy() - ref).max() <= 1e-13 * np.abs(ref).max()
 
 
+def test_band_solve_quotients_are_divisions():
+    """Diagonal systems, whose solution is one quotient an entry, over the range in which
+    the solve multiplies by the pivot's reciprocal and corrects (pivots within 2^+-900,
+    here 2^+-400, and right-hand sides above 2^-960) and past it (2^950, divided): the same
+    bits as the division.  The correction misses the rounding of at most one quotient
+    in some 2^50 (those that close to the middle of two numbers); 2e6 are taken."""
+    import torch
+    from magic_amd import _lib
+    from magic_amd import algebra as A
+    from magic_amd.device import ptr, stream_handle
+    rng = np.random.default_rng(6)
+    n, nl, L = 512, 8, 2048
+    signed = lambda shape, e: rng.choice((-1.0, 1.0), shape) * rng.uniform(1.0, 2.0, shape) * \
+        2.0 ** rng.integers(-e, e, shape)
+    for d in (signed((nl, n), 400), signed((nl, n), 20) * 2.0 ** 930):
+        abd = np.zeros((nl, 3, n))
+        abd[:, 1] = d       # kl = 1, ku = 0 with empty off-diagonals
+        gabd, gpiv, _ = A.prepare_band_batched(torch.from_numpy(abd), n, 1, 0)  # (info: tiny pivots)
+        assert np.array_equal(gabd.cpu().numpy()[:, 1], d)
+        lidx = np.sort(rng.integers(0, nl, L)).astype(np.int32)
+        rhs = signed((L, n), 400) + 1j * signed((L, n), 400)
+        t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()
+        li, r = t(lidx), t(rhs)
+        out = torch.empty_like(r)
+        gp = gpiv.cuda().to(torch.int32).contiguous()
+        _lib.call("mh_band_solve", ptr(gabd), ptr(gp), None, None, ptr(li), None, ptr(r), ptr(out), L, n,
+                  1, 0, stream_handle())
+        x = out.cpu().numpy()
+        assert np.array_equal(x.real, rhs.real / d[lidx]) and np.array_equal(x.imag, rhs.imag / d[lidx])
+
+
 def test_band_singular_info_and_single_solve():
     import torch
     from magic_amd import algebra as A

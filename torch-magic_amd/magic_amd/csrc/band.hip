@@ -192,8 +192,11 @@ extern "C" int mh_band_factor(double* abd, int* pivot, int* info, int n, int kl,
 // unconditional clamped loads, after the stores of the tile before (a wait for the
 // loads would otherwise cover the stores); and the pivots' reciprocals are formed
 // when the factors are staged, so that a step of the back substitution waits for a
-// product and its correction, which give the correctly rounded quotient, instead
-// of a division.  28 KB of LDS at most and below 256 registers: five waves fit on a
+// product and its correction instead of a division.  The product is within 1.5 units in
+// the last place (the reciprocal and itself rounded) and its remainder exact but for
+// the last of 54 bits, so the corrected quotient has the division's bits unless it lies
+// within about 2^-50 of the middle of two numbers; and unless the remainder is
+// subnormal (right-hand sides below 2^-960), where it may be off by one unit.  28 KB of LDS at most and below 256 registers: five waves fit on a
 // CU, and 1028 waves are resident at once (with 35 KB or more registers four would
 // have waited for the rest: 390 us).  l_max = 255, n = 512, kl = ku = 3: 407 us ->
 // 280 us (1.1 GB in four passes: 3.9 TB/s of a copy's 5.5), kl = ku = 2: 356 -> 260;
