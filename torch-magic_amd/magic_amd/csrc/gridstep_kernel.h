@@ -225,24 +225,26 @@ struct Ctx {
 };
 
 // One LDS pass of radix R.  Input groups (Ns) and output groups (Ns*R) are padded
-// by the rule of pads() (a group of one, the packed spectrum, has none).
-template <int R, typename T, bool PAD>
+// by the rule of pads() (a group of one, the packed spectrum, has none).  RT: Ns and nb
+// are known at run time only; the two index forms give the compiler less to keep in
+// registers on either side (compiled plans lose 0.6 % with the other, run-time ones 3 to 5 %).
+template <int R, typename T, bool PAD, bool RT = false>
 __device__ __forceinline__ void stage_mid(const Geo& g, const GridArgs& a, int win, int wout, int Ns,
                                           double dir, int nrows) {
   typedef typename vec2<T>::type V;
   const int nb = g.Mh / R, tstep = g.Mh / (Ns * R);
   const bool pin = PAD && pads(Ns), pout = PAD && pads(Ns * R);
-  const int rstep = pin ? nb + nb / Ns : nb;
+  const int rstep = pin ? nb + nb / Ns : nb, gstep = Ns * R + (pout ? 1 : 0);
   const V* tw = ltw<T>(g);
   const V* in = lbuf<T>(g, win);
   V* out = lbuf<T>(g, wout);
   for (int idx = threadIdx.x; idx < nrows * nb; idx += g.threads) {
     const int row = idx / nb, bf = idx - row * nb;
-    const int k = bf % Ns;
-    const V* src = in + row * g.LS + (pin ? bf / Ns : 0);
+    const int gr = RT ? 0 : Ns == 1 ? bf : bf / Ns, k = RT ? bf % Ns : bf - gr * Ns;
+    const V* src = in + row * g.LS + (RT ? 0 : bf + (pin ? gr : 0));
     V v[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = src[bf + r * rstep];
+    for (int r = 0; r < R; ++r) v[r] = RT ? src[bf + r * nb] : src[r * rstep];
     if (Ns > 1) {
       // powers of w by products from one table value (exp(-i...); the inverse
       // conjugates), for radix 8 from w and w^2, so that none is more than
@@ -272,7 +274,7 @@ __device__ __forceinline__ void stage_mid(const Geo& g, const GridArgs& a, int w
       }
     }
     dft_any<R>(v, dir);
-    V* dst = out + row * g.LS + (bf / Ns) * Ns * R + (pout ? bf / Ns : 0) + k;
+    V* dst = out + row * g.LS + (RT ? (bf / Ns) * Ns * R : gr * gstep) + k;
     if constexpr (sizeof(T) == 4 && (R == 2 || R == 4)) {
       if (Ns == 1) {
         // consecutive outputs from an even element: 16-byte stores of pairs
@@ -294,10 +296,10 @@ __device__ __forceinline__ void stage_mid_rt(const Geo& g, const GridArgs& a, in
                                              int Ns, double dir, int nrows) {
   if (WIDE && R == 8) {
     if constexpr (WIDE) stage_mid<8, T, WIDE>(g, a, win, wout, Ns, dir, nrows);
-  } else if (R == 4) stage_mid<4, T, WIDE>(g, a, win, wout, Ns, dir, nrows);
-  else if (R == 2) stage_mid<2, T, WIDE>(g, a, win, wout, Ns, dir, nrows);
-  else if (R == 3) stage_mid<3, T, WIDE>(g, a, win, wout, Ns, dir, nrows);
-  else stage_mid<5, T, WIDE>(g, a, win, wout, Ns, dir, nrows);
+  } else if (R == 4) stage_mid<4, T, WIDE, !WIDE>(g, a, win, wout, Ns, dir, nrows);
+  else if (R == 2) stage_mid<2, T, WIDE, !WIDE>(g, a, win, wout, Ns, dir, nrows);
+  else if (R == 3) stage_mid<3, T, WIDE, !WIDE>(g, a, win, wout, Ns, dir, nrows);
+  else stage_mid<5, T, WIDE, !WIDE>(g, a, win, wout, Ns, dir, nrows);
 }
 
 // Inverse stages 0 .. nst-2 of a compiled plan (S = stage, NS = its Ns).

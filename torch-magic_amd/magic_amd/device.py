@@ -204,7 +204,8 @@ class Resolution:
         a.Bout = Bout
         a.waves, a.nct = int(waves), int(nct)
         a.minc = self.p.minc
-        a.lcf, a.l_max = ptr(self.d["lcf"]), self.p.l_max
+        if prec == 0:
+            a.lcf, a.l_max = ptr(self.d["lcf"]), self.p.l_max
         _lib.call("mh_leg_synth", 1 if vector else 0, _lib.ref(a), self.M, stream_handle())
 
     def analysis(self, F, Bin, B, comps, outS, outT, ldo, vector: bool, prec=0, waves=0):
@@ -237,7 +238,8 @@ class Resolution:
         a.tiles, a.ntiles = ptr(self.d[f"ana_tiles_{w}"]), self.lay[f"n_ana_tiles_{w}"]
         a.waves = 0 if prec == 0 else w
         a.n_m, a.minc = self.M, self.p.minc
-        a.lcf, a.l_max = ptr(self.d["lcf"]), self.p.l_max
+        if prec == 0:
+            a.lcf, a.l_max = ptr(self.d["lcf"]), self.p.l_max
         _lib.call("mh_leg_analysis", 1 if vector else 0, _lib.ref(a), stream_handle())
 
     def fft(self, forward: bool, F, FB, G, ncomp, B, comp_scale=None):
