@@ -392,6 +392,91 @@ def test_fp64_work_splits_give_identical_results(l_max, B):
             assert (o[:, 0] == 5.0).all() and (o[:, 8:] == 5.0).all() and (o[:, 1:8] != 5.0).all()
 
 
+def _long_double_vector_sums(th, l_max, S, T, ft, fp):
+    """In long double, from the same nodes: the Fourier rows (M, T, B) of the vector
+    synthesis of S and T, and S, T of the vector analysis of the Fourier rows ft, fp
+    (weighted by 1/sin^2), by the products with P and sin(theta) dP (the recurrence of the
+    tables)."""
+    LD = np.longdouble
+    c, s, w = (np.asarray(th[k], dtype=LD) for k in ("cos_n", "sin_n", "w_n"))
+    H, M = c.size, l_max + 1
+    rows = np.zeros((2, M, 2 * H, S.shape[1]), np.clongdouble)
+    sol = np.zeros((2, *S.shape), np.clongdouble)
+    r = lambda a, b: np.sqrt(LD(a) / LD(b))
+    start = 0
+    for m in range(M):
+        n = l_max + 1 - m
+        pi = LD("3.14159265358979323846264338327950288")
+        p0, pm1 = np.sqrt(LD(0.25) / pi) * np.ones(H, LD), np.zeros(H, LD)
+        for q in range(1, m + 1):
+            p0 = p0 * s * r(2 * q + 1, 2 * q)
+        P, D = np.zeros((n, H), LD), np.zeros((n, H), LD)
+        for i in range(n):
+            l = m + i
+            up, dn = r((l + 1 - m) * (l + 1 + m), (2 * l + 1) * (2 * l + 3)), \
+                r((l - m) * (l + m), (2 * l - 1) * (2 * l + 1)) if l > m else LD(0)
+            p1 = (c * p0 - dn * pm1) / up
+            P[i], D[i] = p0, l * up * p1 - (l + 1) * dn * pm1
+            pm1, p0 = p0, p1
+        sl = slice(start, start + n)
+        start += n
+        for e in (0, 1):        # parity of l - m: P keeps it across the equator, dP flips it
+            a, b = S[sl][e::2], T[sl][e::2]
+            q, d = P[e::2].T, D[e::2].T
+            pt, dt = 1j * m * (q @ b), d @ a
+            pp, dp = 1j * m * (q @ a), -(d @ b)
+            sg = 1 - 2 * e
+            rows[0, m, 0::2] += pt + dt
+            rows[0, m, 1::2] += sg * pt - sg * dt
+            rows[1, m, 0::2] += pp + dp
+            rows[1, m, 1::2] += sg * pp - sg * dp
+            fold = lambda f, g: (2 * pi * w)[:, None] * (f[m, 0::2] + g * f[m, 1::2])
+            l = np.arange(m, l_max + 1)[e::2].astype(LD)
+            inv = np.where(l > 0, 1 / np.maximum(l * (l + 1), 1), 0)[:, None]
+            sol[0, sl][e::2] = inv * (d.T @ fold(ft, -sg) - 1j * m * (q.T @ fold(fp, sg)))
+            sol[1, sl][e::2] = inv * (-(d.T @ fold(fp, -sg)) - 1j * m * (q.T @ fold(ft, sg)))
+    return rows, sol
+
+
+@pytest.mark.parametrize("l_max", [33, 85])
+def test_fp64_vector_transforms_row_by_row(l_max):
+    """The FP64 vector transforms combine neighbouring degrees where the oracle multiplies
+    by sin(theta) dP; a cancellation in that would show in single latitudes near the
+    poles or single degrees, not in the largest value.  Errors against long double sums:
+    every latitude (synthesis) and every degree (analysis) within 6 times the oracle's
+    of that row, or of a few roundings of the row's largest value (both come from the
+    rounding of the tables, largest of a few hundred values a row; the ratio is below 3)."""
+    import scipy.fft
+    torch = _torch()
+    from magic_amd.params import Params
+    from magic_amd.device import Resolution
+    from magic_amd.sht import SHT
+    res = Resolution(Params({"l_max": l_max, "n_r_max": 9}))
+    sht, osht = SHT(res), _oracle_sht(l_max)
+    S, T = (_rand_spec(res.L, 3, res.maps, k) for k in (21, 22))
+    S[0] = T[0] = 0.0
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    four = lambda g: scipy.fft.rfft(np.asarray(g, np.longdouble), axis=2, norm="forward")[
+        :, :, :res.M].transpose(2, 1, 0)
+    _, ot, op = osht.torpol_to_spat(0 * S, S, T)
+    gpu = [x.cpu().numpy() for x in sht.torpol_to_spat(dev(0 * S), dev(S), dev(T))[1:]]
+    ost2 = (1 / np.asarray(res.th["sin_grid"], np.longdouble) ** 2)[None, :, None]
+    rows, sol = _long_double_vector_sums(res.th, l_max, S, T, four(ot) * ost2, four(op) * ost2)
+    eps = np.finfo(float).eps
+    for a, b, ref in zip(gpu, (ot, op), rows):
+        err = [np.abs(four(g) - ref).max(axis=(0, 2)) for g in (a, b)]
+        bound = 6 * np.maximum(err[1], 4 * eps * np.abs(ref).max(axis=(0, 2)))
+        print("synthesis", l_max, float((err[0] / np.maximum(err[1], bound / 6)).max()))
+        assert (err[0] <= bound).all(), (err[0] / bound).max()
+    l = res.maps["l"]
+    by_l = lambda x: np.array([np.abs(x[l == k]).max() for k in range(1, l_max + 1)])
+    for a, b, ref in zip(sht.spat_to_sphertor(dev(ot), dev(op)), osht.spat_to_sphertor(ot, op), sol):
+        err = [by_l(v - ref) for v in (a.cpu().numpy(), b)]
+        bound = 6 * np.maximum(err[1], 4 * eps * by_l(ref))
+        print("analysis", l_max, float((err[0] / np.maximum(err[1], bound / 6)).max()))
+        assert (err[0] <= bound).all(), (err[0] / bound).max()
+
+
 def test_fp64_resolution_holds_no_derivative_tables():
     """FP64 transforms read the P_lm tables alone, so a resolution keeps the other two
     only as the FP32 and BF16 copies of a mixed run."""
