@@ -193,10 +193,11 @@ def rowop_wide(run) -> int:
 
 
 def grid_key(res, N: int, fprec: int, l_mag: bool) -> str:
-    # a choice holds for the kernels it was timed with: files written before the radix-8
-    # and batched FP64 plans hold 4 levels where 1 is the best now (l_max = 85, 49 levels:
-    # 231 against 109 us), so the key names the kernels' generation
-    return f"{_device_name(res)}|grid_step/2|Mh={res.Mh}|T={res.T}|M={res.M}|N={N}|fprec={fprec}|mag={int(l_mag)}"
+    # a choice holds for the kernels it was timed with, so the key names their generation:
+    # files written before the compiled own block of n_phi/2 = 256 hold two levels there,
+    # 137 against 130 us in FP32 (33 levels), and those before the batched FP64 plans four
+    # levels at 128, 82 against 79 us
+    return f"{_device_name(res)}|grid_step/3|Mh={res.Mh}|T={res.T}|M={res.M}|N={N}|fprec={fprec}|mag={int(l_mag)}"
 
 
 def grid_level_block(res, N: int, p, fdtype=torch.float64, bufs=None, reps: int = 3) -> int:
