@@ -54,16 +54,17 @@ NOISE = dict(seed=20261202, amp=1e-4)
 # rocprofv3 FETCH_SIZE / WRITE_SIZE passes scaled by a 256 MiB copy (FETCH x 2,
 # WRITE x 1); see profiles/hbm_traffic_l383_nr97_pmc.md.  Grid-step entries are
 # keyed by the tuner's radial levels per workgroup (0: the plan's own block, four
-# levels for the FP32 grid step at n_phi = 1152; the FP64 step chose one); other
-# level blocks have no measured figure (traffic null).  The FP32 Legendre entries
-# ("mixed") are from the same kernels profiled before the BF16 headline; the FP64
-# Legendre kernels have no figure.
+# levels at n_phi = 1152); other level blocks have no measured figure (traffic null).
+# The FP32 Legendre entries ("mixed") are from the same kernels profiled before the
+# BF16 headline.
 PMC_TRAFFIC_BYTES = {
-    ("grid_step", "mixed", 0): 2.540e9 + 1.791e9,
-    ("grid_step", "fp64", 1): 5.861e9 + 4.554e9,
-    ("leg_syn_vec", "mixed_bf16x3"): 3.444e9 + 2.171e9,
+    ("grid_step", "mixed", 0): 2.522e9 + 1.816e9,
+    ("grid_step", "fp64", 0): 6.246e9 + 3.155e9,
+    ("leg_syn_vec", "fp64"): 1.723e9 + 4.344e9,
+    ("leg_syn_vec", "mixed_bf16x3"): 3.446e9 + 2.174e9,
     ("leg_syn_vec", "mixed"): 4.196e9 + 2.192e9,
-    ("leg_ana_vec", "mixed_bf16x3"): 1.640e9 + 0.601e9,
+    ("leg_ana_vec", "fp64"): 2.650e9 + 0.639e9,
+    ("leg_ana_vec", "mixed_bf16x3"): 1.645e9 + 0.601e9,
     ("leg_ana_vec", "mixed"): 1.414e9 + 0.599e9,
 }
 
