@@ -195,7 +195,8 @@ typedef struct {
   double LFfac, cf2, af2;
   int l_mag, alf_damp;
   unsigned long long* cfl; /* 2N per-level maxima (bit patterns of doubles) */
-  int rb;  /* radial levels per workgroup: 0 = the most the FFT plan fits, else 1..that */
+  int rb;  /* radial levels per workgroup: 0 = the most the FFT plan fits, else 1..that (lengths
+              with a compiled plan run 1, 2 or the most, and take 2 for the blocks between) */
   int pad;
 } MhGridArgs;
 
