@@ -531,11 +531,11 @@ def test_fp64_legendre_rows_past_32_bit_offsets():
     torch.cuda.empty_cache()
 
 
-@pytest.mark.parametrize("Mh", [2, 3, 5, 12, 24, 30, 45, 48, 64, 72, 81, 90, 96, 100, 128, 150, 192,
+@pytest.mark.parametrize("Mh", [2, 3, 5, 12, 24, 30, 45, 48, 54, 64, 72, 81, 90, 96, 100, 128, 150, 192,
                                 225, 288, 300, 384, 400, 500, 576, 648, 720, 768, 800, 1000])
 def test_fft_lengths_match_numpy(Mh):
     """mh_fft both ways for compiled, run-time, short and long (> 768) plans (the
-    workgroup's passes below 100 but for two-pass rows: 72, 81), odd and even half
+    workgroup's passes below 50, and with a factor 5 below 100), odd and even half
     lengths, batches that do not fill a workgroup's rows, orders up to Mh; error of a
     few roundings per pass against numpy."""
     torch = _torch()

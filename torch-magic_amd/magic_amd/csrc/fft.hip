@@ -94,16 +94,15 @@ constexpr bool wave_compiled(int Mh) {
   }
 }
 
-// Whether rows of length Mh, `nstage` radix-2 to 5 passes, are transformed by single
-// waves: compiled plans, run-time plans from 100 on, and below that those with half the
-// passes (72: 9 x 8 for 4 x 2 x 3 x 3).  Short rows are a few elements a lane, and the
-// run-time passes' index arithmetic costs more than the workgroup's barriers that they
-// save (k_fft_inverse -> k_wfft_inverse, 8 columns: 30 5.7 -> 7.5 us, 60 7.3 -> 7.5, 80 8.3 ->
-// 9.0, 90 10.0 -> 10.4; 72 9.1 -> 7.0, 100 9.9 -> 8.0, 120 12.0 -> 7.8).
-constexpr bool wave_rows(int Mh, int nstage) {
+// Whether rows of length Mh are transformed by single waves: compiled plans, and run-time
+// plans from 100 on or, without a factor 5, from 50 on.  Shorter rows are a few elements a
+// lane, and the run-time passes' index arithmetic costs more than the workgroup's
+// barriers that they save; radix 9 and 8 save a pass or two at 54 and 72, radix 5 none
+// (k_fft_inverse -> k_wfft_inverse, 8 columns: 30 5.7 -> 7.5 us, 36 6.0 -> 6.6, 60 7.3 -> 7.5, 80
+// 8.3 -> 9.0, 90 10.0 -> 10.4; 54 8.3 -> 7.5, 72 9.1 -> 7.0, 100 9.9 -> 8.0, 120 12.0 -> 7.8).
+constexpr bool wave_rows(int Mh) {
   if (wave_compiled(Mh)) return true;
-  const int nst = make_wplan(Mh).nst;
-  return nst > 0 && (Mh >= 100 || 2 * nst <= nstage);
+  return (Mh >= 100 || (Mh >= 50 && Mh % 5 != 0)) && make_wplan(Mh).nst > 0;
 }
 
 // Geometry and plan of a launch: compile-time constants when MH > 0.
@@ -454,7 +453,7 @@ extern "C" int mh_fft(int forward, const MhFftArgs* args, void* stream) {
   if (prod != a.Mh) return MH_EINVAL;
   const size_t lds = 2ull * a.RB * a.Mh * sizeof(double2);
   if (lds > 160 * 1024) return MH_EINVAL;
-  if (wave_rows(a.Mh, a.nstage)) {
+  if (wave_rows(a.Mh)) {
     if ((long)a.B * a.T * a.ncomp >= 0x7fffffffL) return MH_EINVAL;
     WPlan p = make_wplan(a.Mh);
     while (p.rsh > 0 && (p.RB >> 1) >= a.B) p.RB = 1 << --p.rsh;  // no rows past a short batch
